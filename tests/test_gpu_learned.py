@@ -175,6 +175,30 @@ def test_block_sor_and_residual(torch_gpu):
     assert np.abs(e - v).max() < 1e-10
 
 
+@pytest.mark.parametrize("blocks,sweeps,omega,start", [(1, 0, 1.3, True), (1, 1, 1.0, True),
+                                                        (3, 2, 1.9, False), (5, 33, 0.7, True)])
+def test_block_sor_from_a_start_matches_oracle(torch_gpu, blocks, sweeps, omega, start):
+    """Sweep counts from none, under- and over-relaxation, with and without an
+    initial iterate.  An update is seven rounded terms in either order, so the
+    bound is 64 units of rounding per sweep of the largest value met (about ten
+    terms an update in each of the two, the oracle cancelling diag e)."""
+    torch = torch_gpu
+    from samrai_amd import learned as SL
+    _say("block SOR from a start: %d blocks, %d sweeps" % (blocks, sweeps))
+    rng = np.random.default_rng(blocks + sweeps)
+    h = 1.0 / 48
+    shapes = [(16, 16, 16), (16, 16, 17), (16, 17, 16), (17, 16, 16)]
+    r, dx, dy, dz = (rng.standard_normal((blocks,) + s) for s in shapes)
+    dx, dy, dz = np.exp(dx), np.exp(dy), np.exp(dz)
+    e0 = rng.standard_normal(r.shape) if start else None
+    dev = [torch.from_numpy(a).cuda() for a in (r, dx, dy, dz)]
+    e = SL.block_sor(torch, *dev, h, sweeps, omega,
+                     None if e0 is None else torch.from_numpy(e0).cuda()).cpu().numpy()
+    eo = L.block_sor(r, dx, dy, dz, h, sweeps, omega, e0)
+    top = max(np.abs(eo).max(), 0.0 if e0 is None else np.abs(e0).max())
+    assert np.abs(e - eo).max() <= 64 * 2.0 ** -52 * max(1, sweeps) * top
+
+
 def test_training_on_fac_pairs_gains_over_no_network(torch_gpu):
     torch = torch_gpu
     from samrai_amd import learned as SL
