@@ -108,6 +108,18 @@ void launch_box_side(const LevelGeom& L, const double* const* x, int g, int a, d
                      const BoxLevel& G, int* mismatch, hipStream_t s, int verify,
                      int fp32 = 0);
 
+// ---- levels that fit one work-group's LDS (box_small.hip) ----
+// Does one work-group hold the level (cells, coefficients of A's kind)?
+bool box_lds_fits(const BoxLevel& G, const BoxArrays& A);
+// `sweeps` red-black sweeps in one launch, homogeneous Robin ghosts: u from
+// uin (nullptr: 0) to e0 or e1 by the parity of the sweeps done.  With check,
+// K's early-exit test runs after every sweep (tol, stop, sweeps, maxres_out
+// as launch_box_rbgs and launch_box_final_check leave them); without,
+// nothing is done once *K.stop is set.
+void launch_box_lds_rbgs(const BoxLevel& G, const BoxArrays& A, const RobinDev& bc,
+                         const double* uin, double* e0, double* e1, int sweeps,
+                         const BoxCheck& K, int check, hipStream_t s);
+
 // ---- geometric multigrid on a single-rectangle level ----
 // Largest edge of the grid the one-work-group LDS solve accepts, and the
 // number of partial sums launch_mg_sumsq writes.
@@ -132,12 +144,6 @@ void launch_mg_small_solve(const BoxLevel& G, const BoxArrays& A, const RobinDev
 // mg_partials() partial sums of x^2 (x != nullptr) or of the squared residual of u.
 void launch_mg_sumsq(const BoxLevel& G, const BoxArrays& A, const RobinDev& bc, const double* u,
                      const double* x, double* partial, const int* stop, hipStream_t s);
-// `sweeps` red-black sweeps of u in place (from 0 when zero_in) on a level
-// of at most mg_lds_edge() cells per axis, in one work-group with the level
-// in LDS: the values the same number of launch_box_rbgs sweeps leave.
-int mg_lds_edge();
-void launch_mg_lds_sweeps(const BoxLevel& G, const BoxArrays& A, const RobinDev& bc, double* u,
-                          int sweeps, int zero_in, const int* stop, hipStream_t s);
 // *out = the sum of n partials (launch_sum's order), then the
 // relative-residual test of iteration it on rr = out (it < 0: the b = 0 test
 // only), in one launch (nothing once *stop is set).

@@ -911,10 +911,10 @@ void CellPoissonFACOps::mgSweeps(int m, int n, bool zero_in) {
   sfac::BoxCheck K{};
   K.stop = d_mg_flag;
   const sfac::RobinDev bc = robinDev();
-  bool lds = n > 0 && n % 2 == 0;  // even counts end in e[0], as the ping-pong sweeps do
-  for (int d = 0; d < d_h.dim(); ++d) lds = lds && L.G.n[d] <= sfac::mg_lds_edge();
-  if (lds) {
-    sfac::launch_mg_lds_sweeps(L.G, A, bc, L.e[0], n, zero_in ? 1 : 0, d_mg_flag, d_stream);
+  // a level that fits one work-group's LDS: all its sweeps in one launch
+  if (n > 0 && sfac::box_lds_fits(L.G, A)) {
+    sfac::launch_box_lds_rbgs(L.G, A, bc, zero_in ? nullptr : L.e[0], L.e[0], L.e[1], n, K, 0,
+                              d_stream);
     return;
   }
   if (zero_in && n == 0) {
@@ -1057,7 +1057,13 @@ int CellPoissonFACOps::smoothBox(PatchDataSet& e, const PatchDataSet& r, int num
     tl.start = nextEvent();
     hip_check(hipEventRecord(tl.start, d_stream), "hipEventRecord");
   }
-  for (int s = 0; s < num_sweeps; ++s) {
+  // a level that fits one work-group's LDS takes all its sweeps, with the
+  // early-exit test after each, in one launch (a caller's tile shape asks for
+  // the grid-parallel sweep)
+  const bool lds = num_sweeps > 0 && d_box_variant < 0 && sfac::box_lds_fits(G, A);
+  if (lds)
+    sfac::launch_box_lds_rbgs(G, A, bc, B.e[0], B.e[0], B.e[1], num_sweeps, K, check, d_stream);
+  for (int s = 0; s < num_sweeps && !lds; ++s) {
     K.sweep = s;
     A.ein = B.e[s & 1];
     A.eout = B.e[(s + 1) & 1];
@@ -1072,7 +1078,7 @@ int CellPoissonFACOps::smoothBox(PatchDataSet& e, const PatchDataSet& r, int num
     tl.bytes = launch_bytes * num_sweeps;
     d_timed.push_back(tl);
   }
-  if (check && num_sweeps > 0) {
+  if (check && num_sweeps > 0 && !lds) {
     sfac::launch_box_final_check(K, num_sweeps, d_stream);
   }
   // the sweeps done (known on the device when the loop may stop early)

@@ -1,0 +1,95 @@
+"""Coarsest levels that one work-group holds in LDS: sweeps and early exit
+against the patch-wise passes and the grid-parallel sweep, bit for bit."""
+import numpy as np
+import pytest
+
+import hier_cases as hc
+
+pytestmark = pytest.mark.gpu
+
+KEYS = dict(max_cycles=2, residual_tol=1e-300, relative_residual_tol=1e-300, num_pre_sweeps=1,
+            num_post_sweeps=1, coarse_solver_choice="redblack")
+
+
+def one_level(*n):
+    """A domain of n cells in two patches (the last one decides the early
+    exit), cut at an even index in x (2-D colours are patch-relative)."""
+    dim = len(n)
+    hi = tuple(v - 1 for v in n)
+    cut = n[0] // 2 // 2 * 2
+    if cut == 0:
+        boxes = [((0,) * dim, hi)]
+    else:
+        boxes = [((0,) * dim, (cut - 1,) + hi[1:]), ((cut,) + (0,) * (dim - 1), hi)]
+    return dict(name="x".join(map(str, n)), dim=dim, levels=[boxes], ratio=2, dlo=(0,) * dim,
+                dhi=hi)
+
+
+def solve(case, data, spec, keys, fused, variant, bits):
+    from samrai_amd import fac
+    dim = case["dim"]
+    n0 = np.array(case["dhi"]) + 1
+    h = fac.PatchHierarchy(dim, case["dlo"], case["dhi"], [0.0] * 3,
+                           list(n0 / n0.min()) + [1.0] * (3 - dim))
+    h.add_level(1, case["levels"][0])
+    h.finalize()
+    u, f = fac.PatchData(h, 1), fac.PatchData(h, 0)
+    D = fac.PatchData(h, 0, "side") if spec["dvar"] else None
+    C = fac.PatchData(h, 0) if spec["cmode"] == 2 else None
+    for p in range(len(case["levels"][0])):
+        f.put(0, p, data["f"][0][p])
+        if C is not None:
+            C.put(0, p, data["C"][0][p])
+        if D is not None:
+            for a in range(dim):
+                D.put(0, p, data["D"][0][p][a], axis=a)
+    s = fac.CellPoissonFACSolver(h, **dict(KEYS, **keys))
+    if D is not None:
+        s.set_d_patch_data(D)
+    if C is not None:
+        s.set_c_patch_data(C)
+    elif spec["cmode"] == 1:
+        s.set_c_constant(-0.7)
+    bc = hc.bc_robin(dim) if spec["robin"] else hc.BC_DIRICHLET
+    s.set_boundaries(bc["a"][:2 * dim], bc["b"][:2 * dim], bc["g"][:2 * dim])
+    s.initialize_solver_state(u, f)
+    s.set_coarse_precision(bits)
+    s.set_fused_coarsest(fused, variant)
+    s.solve_system(u, f)
+    out = [u.get(0, p) for p in range(len(case["levels"][0]))]
+    e, r = s.internal_vector("e"), s.internal_vector("r")
+    e.fill(0.0)
+    count = s.smooth(e, r, 0, 9, tol=keys["coarse_solver_tolerance"])
+    return out, np.array(s.history()), count
+
+
+# slots per colour and thread 1, 2, 4 and 8, the last sizes that fit
+# (4096 cells with coefficients, 8192 without) and the first that do not,
+# odd rows, one-cell-wide and thin domains
+SIZES = [(3, 2, 2), (1, 5, 7), (9, 10, 11), (13, 17, 15), (16, 16, 16), (17, 16, 16), (32, 16, 16),
+         (34, 16, 16), (2, 40, 40), (5, 3), (31, 23), (64, 64), (65, 64), (90, 91), (128, 64),
+         (130, 64), (300, 9)]
+
+
+@pytest.mark.parametrize("spec", [dict(dvar=False, cmode=0, robin=False),
+                                  dict(dvar=False, cmode=1, robin=True),
+                                  dict(dvar=True, cmode=2, robin=True)],
+                         ids=["constD", "constD-constC-robin", "varD-varC-robin"])
+@pytest.mark.parametrize("n", SIZES, ids=lambda n: "x".join(map(str, n)))
+def test_lds_sweeps_are_bit_identical(gpu_lib, n, spec):
+    """Solution, residual history, sweep count and maximum residual of the
+    early exit equal those of the patch-wise passes; the FP32 coarse solve
+    equals the grid-parallel sweep's.  Sweep counts odd and even, with a
+    tolerance that stops the loop and one that does not."""
+    case = one_level(*n)
+    data = hc.make_data(case, seed=sum(n))
+    for sweeps, tol in ((7, 1e-300), (40, 0.5)):
+        print("lds sweeps", case["name"], spec, sweeps, tol, flush=True)
+        keys = dict(coarse_solver_max_iterations=sweeps, coarse_solver_tolerance=tol)
+        for bits, fused, variant in ((64, False, 0), (32, True, 0)):
+            ref = solve(case, data, spec, keys, fused, variant, bits)
+            got = solve(case, data, spec, keys, True, -1, bits)
+            assert got[2] == ref[2]
+            np.testing.assert_array_equal(got[1], ref[1])
+            for a, b in zip(got[0], ref[0]):
+                np.testing.assert_array_equal(a, b)
