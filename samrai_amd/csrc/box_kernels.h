@@ -120,9 +120,26 @@ void launch_box_lds_rbgs(const BoxLevel& G, const BoxArrays& A, const RobinDev& 
                          const double* uin, double* e0, double* e1, int sweeps,
                          const BoxCheck& K, int check, hipStream_t s);
 
+// The lower part of a multigrid V-cycle in one launch, over the n levels G
+// (each half the one before) with arrays A (r of the first is its right-hand
+// side): pre-sweeps, residual restriction, ..., `last` sweeps from 0 on the
+// smallest, prolongation, post-sweeps; the first level's error from 0
+// (from_input 0) or from e, to e.  columns (the first level's cells): the map
+// from right-hand side to error instead, as a row-major matrix in e.
+// mg_bottom_first: the first of n levels with at most kMGDenseCells cells
+// from which on they fit a work-group (n: none).
+constexpr int kMGDenseCells = 1024;
+int mg_bottom_first(const BoxLevel* G, int n);
+void launch_mg_bottom(const BoxLevel* G, const BoxArrays* A, int n, const RobinDev& bc, int pre,
+                      int post, int last, double* e, int from_input, int columns,
+                      const int* stop, hipStream_t s);
+// e = B f for that matrix of n rows.
+void launch_mg_dense(const double* B, int n, const double* f, double* e, int fp32,
+                     const int* stop, hipStream_t s);
+
 // ---- geometric multigrid on a single-rectangle level ----
-// Largest edge of the grid the one-work-group LDS solve accepts, and the
-// number of partial sums launch_mg_sumsq writes.
+// Edge of the smallest multigrid grid (halving stops there), and the number
+// of partial sums launch_mg_sumsq writes.
 int mg_small_edge();
 int mg_partials();
 // Arrays u, x, fc, ec, ef, Dc, Cc have the precision of A.fp32 (fp32).
@@ -137,10 +154,6 @@ void launch_mg_prolong_add(const BoxLevel& Gc, const RobinDev& bc, const double*
 // Coarse D faces (mean of the fine faces they cover) and C (mean of children).
 void launch_mg_coarsen_coef(const BoxLevel& Gf, const BoxArrays& Af, const BoxLevel& Gc,
                             double* const* Dc, double* Cc, hipStream_t s);
-// u = 0, then `sweeps` red-black sweeps on a grid of at most mg_small_edge()
-// cells per axis, in one work-group.
-void launch_mg_small_solve(const BoxLevel& G, const BoxArrays& A, const RobinDev& bc, double* u,
-                           int sweeps, const int* stop, hipStream_t s);
 // mg_partials() partial sums of x^2 (x != nullptr) or of the squared residual of u.
 void launch_mg_sumsq(const BoxLevel& G, const BoxArrays& A, const RobinDev& bc, const double* u,
                      const double* x, double* partial, const int* stop, hipStream_t s);

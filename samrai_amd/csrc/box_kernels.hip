@@ -573,77 +573,6 @@ k_mg_coarsen_coef(BoxLevel Gf, BoxArraysT<T> Af, BoxLevel Gc, T* Dc0, T* Dc1, T*
 }
 
 constexpr int kMGSmallEdge = 4;
-constexpr int kMGSmallThreads = 64;
-template <int DIM, int EDGE>
-constexpr int mg_lds_size() {
-  return DIM == 3 ? (EDGE + 2) * (EDGE + 2) * (EDGE + 2) : (EDGE + 2) * (EDGE + 2);
-}
-// `sweeps` red-black sweeps of a grid of at most EDGE cells per axis held in
-// LDS (U, mg_lds_size values) by a work-group of NT threads, each thread's
-// cell coefficients and reciprocal diagonals in registers and the Robin
-// ghosts formed inside the updates (the cell is its face ghost's only
-// interior neighbour); u starts from uin (nullptr: 0) and ends in uout.
-// Red <=> (level indices + shift) even, red first, as k_box_rbgs; updates of
-// one colour are independent, so sweeping in place equals its ping-pong
-// tiles bit for bit.
-template <int DIM, bool DVAR, int CMODE, typename T, int NT, int EDGE>
-__device__ inline void mg_lds_block(const BoxLevel& G, const BoxArraysT<T>& A,
-                                    const RobinDev& bc, const T* uin, T* uout, int sweeps,
-                                    T* U) {
-  constexpr int kThreads = NT;
-  constexpr int L = EDGE + 2;
-  constexpr int SY = L, SZ = L * L;
-  constexpr int NMAX = DIM == 3 ? EDGE * EDGE * EDGE : EDGE * EDGE;
-  constexpr int NC = (NMAX + kThreads - 1) / kThreads;
-  const int n0 = G.n[0], n1 = G.n[1], n2 = DIM == 3 ? G.n[2] : 1;
-  const int ncell = n0 * n1 * n2;
-  const int par0 = G.lo[0] + G.lo[1] + (DIM == 3 ? G.lo[2] : 0) + G.shift;
-  for (int q = threadIdx.x; q < mg_lds_size<DIM, EDGE>(); q += kThreads) U[q] = (T)0;
-  __syncthreads();
-  int qc[NC], col[NC], bm[NC];
-  Coef<T> cf[NC];
-  T dudr[NC];
-#pragma unroll
-  for (int v = 0; v < NC; ++v) {
-    const int t = threadIdx.x + v * kThreads;
-    qc[v] = -1;
-    if (t < ncell) {
-      const int i = t % n0, j = (t / n0) % n1, k = DIM == 3 ? t / (n0 * n1) : 0;
-      qc[v] = (i + 1) + SY * (j + 1) + SZ * (DIM == 3 ? k + 1 : 0);
-      col[v] = pos2(par0 + i + j + k);
-      cf[v] = load_coef<DIM, DVAR, CMODE>(G, A, i, j, k);
-      dudr[v] = cell_dudr<DIM, DVAR, CMODE>(cf[v], G, A);
-      // every face of this grid is on the physical boundary
-      bm[v] = (i == 0 ? 1 : 0) | (i == n0 - 1 ? 2 : 0) | (j == 0 ? 4 : 0) |
-              (j == n1 - 1 ? 8 : 0) |
-              (DIM == 3 ? (k == 0 ? 16 : 0) | (k == n2 - 1 ? 32 : 0) : 0);
-      if (uin) U[qc[v]] = uin[t];
-    }
-  }
-  __syncthreads();
-  for (int s = 0; s < sweeps; ++s)
-    for (int colour = 0; colour < 2; ++colour) {
-#pragma unroll
-      for (int v = 0; v < NC; ++v)
-        if (qc[v] >= 0 && col[v] == colour)
-          cell_update<DIM, DVAR, CMODE>(U, qc[v], SY, SZ, SZ, cf[v], G, A, dudr[v], bm[v], &bc);
-      __syncthreads();
-    }
-#pragma unroll
-  for (int v = 0; v < NC; ++v)
-    if (qc[v] >= 0) uout[threadIdx.x + v * kThreads] = U[qc[v]];
-}
-
-// The smallest grid (at most kMGSmallEdge cells per axis): u = 0, then
-// `sweeps` sweeps (mg_lds_block); one wavefront, one cell per lane.
-template <int DIM, bool DVAR, int CMODE, typename T>
-__global__ void __launch_bounds__(kMGSmallThreads)
-k_mg_small_solve(BoxLevel G, BoxArraysT<T> A, RobinDev bc, T* u, int sweeps, const int* stop) {
-  __shared__ T U[mg_lds_size<DIM, kMGSmallEdge>()];
-  if (*stop) return;
-  mg_lds_block<DIM, DVAR, CMODE, T, kMGSmallThreads, kMGSmallEdge>(G, A, bc, nullptr, u, sweeps,
-                                                                    U);
-}
 
 // Partial sums of the squared residual (x == nullptr) or of x^2 over a
 // level, one per work-group of a fixed grid.
@@ -827,17 +756,6 @@ struct RestrictRun {
 };
 
 template <int DIM, bool DVAR, int CMODE>
-struct SmallRun {
-  template <typename T>
-  static void run(const BoxLevel& G, const BoxArraysT<T>& A, const RobinDev& bc, T* u,
-                  int sweeps, const int* stop, hipStream_t s) {
-    hipLaunchKernelGGL((k_mg_small_solve<DIM, DVAR, CMODE, T>), dim3(1), dim3(kMGSmallThreads), 0, s, G,
-                       A, bc, u, sweeps, stop);
-    check_launch();
-  }
-};
-
-template <int DIM, bool DVAR, int CMODE>
 struct SumsqRun {
   template <typename T>
   static void run(const BoxLevel& G, const BoxArraysT<T>& A, const RobinDev& bc, const T* u,
@@ -903,12 +821,6 @@ void launch_mg_coarsen_coef(const BoxLevel& Gf, const BoxArrays& Af, const BoxLe
   } else {
     mg_coarsen<double>(Gf, typed<double>(Af), Gc, Dc, Cc, s);
   }
-}
-
-void launch_mg_small_solve(const BoxLevel& G, const BoxArrays& A, const RobinDev& bc, double* u,
-                           int sweeps, const int* stop, hipStream_t s) {
-  if (A.fp32) dispatch3<SmallRun>(G, typed<float>(A), bc, as<float>(u), sweeps, stop, s);
-  else dispatch3<SmallRun>(G, typed<double>(A), bc, u, sweeps, stop, s);
 }
 
 void launch_mg_sumsq(const BoxLevel& G, const BoxArrays& A, const RobinDev& bc, const double* u,

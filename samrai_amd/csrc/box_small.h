@@ -212,7 +212,9 @@ __device__ inline void small_load(const BoxLevel& G, const BoxArraysT<T>& A, con
                         (j == n1 - 1 ? 8 : 0) |
                         (DIM == 3 ? (k == 0 ? 16 : 0) | (k == n2 - 1 ? 32 : 0) : 0) |
                         (lp ? 128 : 0) | (i + n0 * (j + n1 * k)) << 8;
-        q.k[c][v] = load_coef<DIM, DVAR, CMODE>(G, A, i, j, k);
+        q.k[c][v] = load_coef<DIM, DVAR, 0>(G, A, i, j, k);
+        // a constant C may come as C mode 2 without an array (k_mg_bottom)
+        if (CMODE == 2) q.k[c][v].c = A.C ? A.C[i + n0 * (j + n1 * k)] : (T)A.cconst;
       }
     }
   }

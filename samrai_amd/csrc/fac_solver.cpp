@@ -822,6 +822,7 @@ sfac::BoxArrays CellPoissonFACOps::gatherBox(PatchDataSet& e, const PatchDataSet
 
 namespace {
 constexpr int kMGPre = 2, kMGPost = 2, kMGSmallSweeps = 60, kMGLastSweeps = 64;
+constexpr int kMGDenseCycles = 4;  // V-cycles from which on the matrix pays
 }
 
 void CellPoissonFACOps::releaseMG() {
@@ -831,6 +832,8 @@ void CellPoissonFACOps::releaseMG() {
       if (p) (void)hipFree(p);
   }
   d_mg.clear();
+  if (d_mg_dense) (void)hipFree(d_mg_dense);
+  d_mg_dense = nullptr;
   if (d_mg_partial) (void)hipFree(d_mg_partial);
   if (d_mg_scal) (void)hipFree(d_mg_scal);
   if (d_mg_flag) (void)hipFree(d_mg_flag);
@@ -884,6 +887,13 @@ void CellPoissonFACOps::setupMG() {
   d_mg_small_direct = d_mg.size() > 1;
   for (int d = 0; d < dim; ++d)
     if (d_mg.back().G.n[d] > edge) d_mg_small_direct = false;
+  d_mg_boxes.clear();
+  for (const MGLevel& L : d_mg) d_mg_boxes.push_back(L.G);
+  d_mg_bottom = sfac::mg_bottom_first(d_mg_boxes.data(), (int)d_mg_boxes.size());
+  if (d_mg_bottom > 0 && d_mg_bottom < (int)d_mg.size()) {
+    const size_t n = mgCells(d_mg_bottom);
+    hip_check(hipMalloc(&d_mg_dense, sizeof(double) * n * n), "hipMalloc(mg)");
+  }
   hip_check(hipMalloc(&d_mg_partial, sizeof(double) * sfac::mg_partials()), "hipMalloc(mg)");
   hip_check(hipMalloc(&d_mg_scal, sizeof(double) * 4), "hipMalloc(mg)");
   hip_check(hipMalloc(&d_mg_flag, sizeof(int) * 2), "hipMalloc(mg)");
@@ -929,13 +939,31 @@ void CellPoissonFACOps::mgSweeps(int m, int n, bool zero_in) {
   }
 }
 
+int CellPoissonFACOps::mgCells(int m) const {
+  const sfac::BoxLevel& G = d_mg[m].G;
+  return G.n[0] * G.n[1] * (d_h.dim() == 3 ? G.n[2] : 1);
+}
+
+// The lower part of the V-cycle (levels d_mg_bottom on): its error into e,
+// or with columns its matrix.
+void CellPoissonFACOps::mgBottom(int columns, double* e) {
+  const int m = d_mg_bottom;
+  std::vector<sfac::BoxArrays> A;
+  for (int l = m; l < (int)d_mg.size(); ++l) A.push_back(mgArrays(l));
+  sfac::launch_mg_bottom(d_mg_boxes.data() + m, A.data(), (int)A.size(), robinDev(), kMGPre,
+                         kMGPost, d_mg_small_direct ? kMGSmallSweeps : kMGLastSweeps, e,
+                         columns == 0 && m == 0, columns, d_mg_flag, d_stream);
+}
+
 void CellPoissonFACOps::mgVcycle(int m) {
   MGLevel& L = d_mg[m];
   const sfac::RobinDev bc = robinDev();
   const bool last = m + 1 == (int)d_mg.size();
-  if (last && d_mg_small_direct) {
-    sfac::launch_mg_small_solve(L.G, mgArrays(m), bc, L.e[0], kMGSmallSweeps, d_mg_flag,
-                                d_stream);
+  if (m == d_mg_bottom) {
+    if (d_mg_use_dense)
+      sfac::launch_mg_dense(d_mg_dense, mgCells(m), L.f, L.e[0], d_box.fp32, d_mg_flag, d_stream);
+    else
+      mgBottom(0, L.e[0]);
     return;
   }
   // the error of a coarser level starts at 0: its first sweep reads no
@@ -977,6 +1005,11 @@ void CellPoissonFACOps::solveBoxMG(PatchDataSet& e, const PatchDataSet& r) {
   // ||r||^2 into d_mg_scal[1] and the relative-residual test
   sfac::launch_mg_sum_check(d_mg_partial, P, d_mg_scal, d_mg_scal, tol, -1, d_mg_flag,
                             d_mg_flag + 1, d_mg_scal + 2, d_stream);
+  // the lower levels' matrix takes about as long as two passes through them;
+  // formed per solve, since the caller may change the coefficients between
+  // solves (level 0 starts from the last V-cycle's error, not from 0)
+  d_mg_use_dense = d_mg_dense && d_coarse_max >= kMGDenseCycles;
+  if (d_mg_use_dense) mgBottom(mgCells(d_mg_bottom), d_mg_dense);
   for (int it = 0; it < d_coarse_max; ++it) {
     mgVcycle(0);
     sfac::launch_mg_sumsq(d_mg[0].G, mgArrays(0), bc, d_mg[0].e[0], nullptr, d_mg_partial,

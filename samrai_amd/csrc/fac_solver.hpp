@@ -337,6 +337,12 @@ class CellPoissonFACOps : public FACOperatorStrategy {
     double* C = nullptr;
   };
   std::vector<MGLevel> d_mg;  // [0] aliases the box arrays
+  std::vector<sfac::BoxLevel> d_mg_boxes;  // of d_mg
+  int d_mg_bottom = 0;         // first level of the lower part
+  double* d_mg_dense = nullptr;  // its matrix while a solve uses one
+  bool d_mg_use_dense = false;
+  int mgCells(int m) const;
+  void mgBottom(int columns, double* e);
   bool d_mg_small_direct = false;
   bool d_prolong_coarse_filled = false;
   std::vector<int*> d_lwin;  // learned-correction windows per level (device)
