@@ -330,13 +330,15 @@ void launch_tile(const BoxLevel& G, const BoxArraysT<T>& A, const RobinDev& bc, 
   check_launch();
 }
 
-constexpr int kVariants = 9;
+constexpr int kVariants = 13;
 constexpr BoxTile kTiles3[kVariants] = {{32, 8, 8}, {16, 8, 8},  {32, 16, 4},
                                         {64, 4, 4}, {32, 8, 4},  {16, 16, 4},
-                                        {16, 16, 8}, {32, 16, 8}, {24, 8, 8}};
+                                        {16, 16, 8}, {32, 16, 8}, {24, 8, 8},
+                                        {16, 4, 4}, {16, 8, 4}, {8, 8, 4}, {8, 4, 4}};
 constexpr BoxTile kTiles2[kVariants] = {{64, 16, 1}, {32, 16, 1}, {32, 32, 1},
                                         {128, 8, 1}, {64, 8, 1},  {16, 16, 1},
-                                        {64, 16, 1}, {64, 16, 1}, {64, 16, 1}};
+                                        {64, 16, 1}, {64, 16, 1}, {64, 16, 1},
+                                        {16, 8, 1}, {32, 8, 1}, {64, 4, 1}, {8, 8, 1}};
 
 template <int DIM, bool DVAR, int CMODE, typename T>
 void launch_variant(int variant, const BoxLevel& G, const BoxArraysT<T>& A, const RobinDev& bc,
@@ -351,6 +353,10 @@ void launch_variant(int variant, const BoxLevel& G, const BoxArraysT<T>& A, cons
       case 6: launch_tile<3, DVAR, CMODE, 16, 16, 8>(G, A, bc, homogeneous, K, s); break;
       case 7: launch_tile<3, DVAR, CMODE, 32, 16, 8>(G, A, bc, homogeneous, K, s); break;
       case 8: launch_tile<3, DVAR, CMODE, 24, 8, 8>(G, A, bc, homogeneous, K, s); break;
+      case 9: launch_tile<3, DVAR, CMODE, 16, 4, 4>(G, A, bc, homogeneous, K, s); break;
+      case 10: launch_tile<3, DVAR, CMODE, 16, 8, 4>(G, A, bc, homogeneous, K, s); break;
+      case 11: launch_tile<3, DVAR, CMODE, 8, 8, 4>(G, A, bc, homogeneous, K, s); break;
+      case 12: launch_tile<3, DVAR, CMODE, 8, 4, 4>(G, A, bc, homogeneous, K, s); break;
       default: launch_tile<3, DVAR, CMODE, 32, 8, 8>(G, A, bc, homogeneous, K, s); break;
     }
   } else {
@@ -360,6 +366,10 @@ void launch_variant(int variant, const BoxLevel& G, const BoxArraysT<T>& A, cons
       case 3: launch_tile<2, DVAR, CMODE, 128, 8, 1>(G, A, bc, homogeneous, K, s); break;
       case 4: launch_tile<2, DVAR, CMODE, 64, 8, 1>(G, A, bc, homogeneous, K, s); break;
       case 5: launch_tile<2, DVAR, CMODE, 16, 16, 1>(G, A, bc, homogeneous, K, s); break;
+      case 9: launch_tile<2, DVAR, CMODE, 16, 8, 1>(G, A, bc, homogeneous, K, s); break;
+      case 10: launch_tile<2, DVAR, CMODE, 32, 8, 1>(G, A, bc, homogeneous, K, s); break;
+      case 11: launch_tile<2, DVAR, CMODE, 64, 4, 1>(G, A, bc, homogeneous, K, s); break;
+      case 12: launch_tile<2, DVAR, CMODE, 8, 8, 1>(G, A, bc, homogeneous, K, s); break;
       default: launch_tile<2, DVAR, CMODE, 64, 16, 1>(G, A, bc, homogeneous, K, s); break;
     }
   }

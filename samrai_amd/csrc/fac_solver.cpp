@@ -935,8 +935,19 @@ void CellPoissonFACOps::mgSweeps(int m, int n, bool zero_in) {
   for (int s = 0; s < n; ++s) {
     A.ein = (s == 0 && zero_in) ? nullptr : L.e[s & 1];
     A.eout = L.e[(s + 1) & 1];
-    sfac::launch_box_rbgs(L.G, A, bc, 1, K, d_box.variant, d_stream);
+    sfac::launch_box_rbgs(L.G, A, bc, 1, K, mgVariant(m), d_stream);
   }
+}
+
+// Tile shape of multigrid level m's sweeps: the tuned one on the finest level
+// (or the caller's); below it a sweep is latency, shortest with tiles small
+// enough for more work-groups than compute units (32^3 variable D: 16x4x4
+// 5.8 us, 16x8x8 7.9; 64^3: 16x8x4 7.6, 16x8x8 8.2, 16x4x4 8.3; 2-D 124 x 92:
+// 16x8 3.9, 16x16 4.1).
+int CellPoissonFACOps::mgVariant(int m) const {
+  if (m == 0 || d_box_variant >= 0) return d_box.variant;
+  if (d_h.dim() == 2) return sfac::kBoxTile16x8;
+  return mgCells(m) <= 100000 ? sfac::kBoxTile16x4x4 : sfac::kBoxTile16x8x4;
 }
 
 int CellPoissonFACOps::mgCells(int m) const {

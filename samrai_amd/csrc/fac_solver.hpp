@@ -342,6 +342,7 @@ class CellPoissonFACOps : public FACOperatorStrategy {
   double* d_mg_dense = nullptr;  // its matrix while a solve uses one
   bool d_mg_use_dense = false;
   int mgCells(int m) const;
+  int mgVariant(int m) const;
   void mgBottom(int columns, double* e);
   bool d_mg_small_direct = false;
   bool d_prolong_coarse_filled = false;
