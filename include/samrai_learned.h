@@ -90,6 +90,10 @@ int sfac_learned_features(void* net, const double* r, const double* logd, double
 int sfac_learned_forward(void* net, int nblocks, hipStream_t stream);
 /* e = omega * s * prediction (FP64), after features + forward. */
 int sfac_learned_correction(void* net, double omega, double* e, int nblocks, hipStream_t stream);
+/* features + forward + correction in one launch: the same buffers and state
+ * afterwards. */
+int sfac_learned_apply(void* net, const double* r, const double* logd, double h, double omega,
+                       double* e, int nblocks, hipStream_t stream);
 /* Loss mean((prediction - target / s)^2) and the gradients of every layer,
  * after features + forward on the same blocks. */
 int sfac_learned_backward(void* net, const double* target, int nblocks, hipStream_t stream);

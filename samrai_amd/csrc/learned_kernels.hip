@@ -22,6 +22,7 @@
 // 3(dy+1) + (dx+1).
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cmath>
 #include <cstdint>
 #include <cstring>
@@ -54,10 +55,15 @@ constexpr int NPAIR = (NTAP + 1) / 2;  // tap pairs per K = 32 MFMA
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 
 __host__ __device__ inline uint16_t f2bf(float f) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  // the conversion instruction rounds to nearest even too
+  return __builtin_bit_cast(uint16_t, (__bf16)f);
+#else
   uint32_t u;
   memcpy(&u, &f, 4);
   u += 0x7fffu + ((u >> 16) & 1u);  // round to nearest even (inputs are finite)
   return (uint16_t)(u >> 16);
+#endif
 }
 __host__ __device__ inline float bf2f(uint16_t h) {
   uint32_t u = (uint32_t)h << 16;
@@ -164,6 +170,285 @@ __global__ __launch_bounds__(256) void k_conv(const uint16_t* __restrict__ x,
         const bool on = bf2f(mask[cell * CH + cx]) > 0.f;
         out[cell * CH + cx] = f2bf(on ? v : 0.f);
       }
+    }
+  }
+}
+
+// ---------------------------------------------------------------------------
+// The three layers in one kernel.
+//
+// Layer by layer the network moves every hidden activation (32 B a cell)
+// through HBM twice and does 14 K = 32 products of 16 cells per layer although
+// the first layer has 2 input channels and the last 1 output channel.  Here a
+// work-group takes a z-slab of a block (the whole block when there are enough
+// of them) and marches through its planes, four of each hidden layer in LDS:
+// step i forms plane i + 2 of the first layer, plane i of the second, the tap
+// products of plane i - 2 of the third and the prediction of plane i - 3, all
+// from planes of earlier steps, so that one barrier a step is enough (it
+// waits for LDS only, the stores drain behind it).  Nothing but the features
+// and the result is in memory.  What bounds it are the LDS reads and, of a
+// block, the latency of its 64 KB of input, which is loaded while the block
+// before it is worked on:
+//   layer 1: K holds 16 taps x 2 channels, so 2 products a row;
+//   layer 2: a fragment (row y', taps dx = -1 and 0 of one dz, or dx = 1 of two)
+//     serves the three output rows y' - 1 .. y' + 1, 5 fragments a row and 15
+//     products (20 fragment reads for the two rows a wave forms, not 28);
+//   layer 3: N holds the 9 (dy, dx) taps, K two dz, 2 products a row; the
+//     prediction is then 9 adds per cell.
+// A correction of 4096 blocks (features, three layers, correction) 1.66 ms as
+// five kernels, 0.58 ms so: 0.49 PFLOP/s of real channels, 1.7 TB/s.
+constexpr int FWD_THREADS = 512;
+constexpr int FP = HB * HB;          // cells of a halo-padded plane
+constexpr int FWD_F = HB * FP;       // words: features, two BF16 a cell, all planes
+constexpr int FWD_H = FP * 2;        // uint4 per plane of 16 channels
+constexpr int FWD_G = FP * 9;        // floats per plane of tap products
+constexpr int FWD_LDS = FWD_F * 4 + 8 * FWD_H * 16 + 2 * FWD_G * 4;  // 129600 B
+
+struct Forward {
+  const uint16_t* x0;    // features (FROM_R false)
+  const double* r;       // residual and log D (nullptr: logd_const), FROM_R
+  const double* logd;
+  double logd_const, h2;
+  uint16_t* x0_out;      // features, scales (FROM_R)
+  double* scale;
+  const uint16_t* w[NLAYER];
+  const float* bias[NLAYER];
+  uint16_t* act[2];      // hidden activations (SAVE)
+  float* pred;
+  double* e;             // omega * scale * prediction (FROM_R)
+  double omega;
+  int nblocks;
+  int* unsaved;          // blocks whose hidden activations were not stored
+  int only_unsaved;      // do nothing unless *unsaved covers the block
+};
+
+// Barrier that orders LDS accesses only.
+__device__ inline void lds_barrier() {
+  asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+}
+
+// SAVE: store the hidden activations (training).  FROM_R: one work-group per
+// block at a time forms its scale and features from the residual and writes
+// the correction; else a work-group takes 16 / slabs planes of a block.
+// Work-group b takes slabs b, b + gridDim.x, ... of all.
+template <bool SAVE, bool FROM_R>
+__global__ __launch_bounds__(FWD_THREADS) void k_forward(Forward P, int slabs) {
+  __shared__ __align__(16) unsigned char lds[FWD_LDS];
+  uint32_t* F = reinterpret_cast<uint32_t*>(lds);
+  uint4* H1 = reinterpret_cast<uint4*>(lds + FWD_F * 4);
+  uint4* H2 = H1 + 4 * FWD_H;
+  float* G = reinterpret_cast<float*>(H2 + 4 * FWD_H);
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int cx = lane & 15, g = lane >> 4, half = g & 1, tsel = g >> 1;
+  const int nwork = P.only_unsaved ? *P.unsaved * slabs : P.nblocks * slabs;
+  if ((int)blockIdx.x >= nwork) return;
+  constexpr int NV = FROM_R ? NCELL / FWD_THREADS : 1;
+  double rv[NV], lv[NV];
+  auto fetch = [&](int b) {  // a block's residual and log D
+    if (FROM_R)
+#pragma unroll
+      for (int k = 0; k < NV; ++k) {
+        const size_t c = (size_t)b * NCELL + threadIdx.x + k * FWD_THREADS;
+        rv[k] = P.r[c];
+        lv[k] = P.logd ? P.logd[c] : P.logd_const;
+      }
+  };
+  fetch(blockIdx.x);
+  for (int q = threadIdx.x; q < FWD_LDS / 16; q += FWD_THREADS)
+    reinterpret_cast<uint4*>(lds)[q] = make_uint4(0u, 0u, 0u, 0u);
+
+  // weights: layer 1 [m], layer 2 [5 kinds][dy], layer 3 [dz pair]
+  bf16x8 w1[2], w2[5][3], w3[2];
+  // layer 1's inputs: taps 16 m + 4 g .. + 3 (two channels each) of the
+  // lane's cell, as offsets in F; the taps past the 27th have zero weights
+  int off1[2][4];
+#pragma unroll
+  for (int m = 0; m < 2; ++m) {
+    uint32_t u[4];
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      const int t = 16 * m + 4 * g + k, tt = min(t, NTAP - 1);
+      u[k] = t < NTAP ? *reinterpret_cast<const uint32_t*>(P.w[0] + (t * CH + cx) * CH) : 0u;
+      off1[m][k] = ((tt / 9) * HB + (tt / 3) % 3 + 2 * wave) * HB + cx + tt % 3;
+    }
+    w1[m] = __builtin_bit_cast(bf16x8, make_uint4(u[0], u[1], u[2], u[3]));
+  }
+#pragma unroll
+  for (int f = 0; f < 5; ++f)
+#pragma unroll
+    for (int dy = 0; dy < 3; ++dy) {
+      // f < 3: dz = f, dx = tsel; f = 3: dz = tsel, dx = 2; f = 4: dz = 2, dx = 2
+      const int dz = f < 3 ? f : (f == 3 ? tsel : 2), dx = f < 3 ? tsel : 2;
+      const int t = dz * 9 + dy * 3 + dx;
+      uint4 v = make_uint4(0u, 0u, 0u, 0u);
+      if (f < 4 || tsel == 0)
+        v = *reinterpret_cast<const uint4*>(P.w[1] + (t * CH + cx) * CH + 8 * half);
+      w2[f][dy] = __builtin_bit_cast(bf16x8, v);
+    }
+#pragma unroll
+  for (int m = 0; m < 2; ++m) {
+    const int dz = m == 0 ? tsel : 2;
+    uint4 v = make_uint4(0u, 0u, 0u, 0u);
+    if (cx < 9 && (m == 0 || tsel == 0))
+      v = *reinterpret_cast<const uint4*>(P.w[2] + ((dz * 9 + cx) * CH) * CH + 8 * half);
+    w3[m] = __builtin_bit_cast(bf16x8, v);
+  }
+  const float b1 = P.bias[0][cx], b2 = P.bias[1][cx], b3 = P.bias[2][0];
+  if (P.unsaved && !P.only_unsaved && threadIdx.x == 0) *P.unsaved = SAVE ? 0 : P.nblocks;
+  const int nz = NB / slabs;
+  const int y0 = 2 * wave;  // this wave's rows
+  uint16_t* h1 = reinterpret_cast<uint16_t*>(H1);
+  uint16_t* h2 = reinterpret_cast<uint16_t*>(H2);
+  lds_barrier();
+
+  for (int work = blockIdx.x; work < nwork; work += gridDim.x) {
+    const int b = work / slabs, z0 = (work % slabs) * nz, zend = z0 + nz;
+    // features of the block into F (interior; the halo stays 0)
+    double scale = 0.0;
+    if (FROM_R) {
+      double* red = reinterpret_cast<double*>(G);  // free here
+      double s2 = 0.0;
+#pragma unroll
+      for (int k = 0; k < NV; ++k) {
+        rv[k] *= P.h2;
+        s2 += rv[k] * rv[k];
+      }
+      for (int o = 32; o > 0; o >>= 1) s2 += __shfl_xor(s2, o, 64);
+      if (lane == 0) red[wave] = s2;
+      lds_barrier();
+      s2 = 0.0;
+#pragma unroll
+      for (int k = 0; k < FWD_THREADS / 64; ++k) s2 += red[k];
+      lds_barrier();
+      if (threadIdx.x < FWD_THREADS / 64) red[threadIdx.x] = 0.0;  // G's halo is read as zeros
+      // a block whose residual is zero (or not finite) gets scale 0 (k_features)
+      const double sq = sqrt(s2 / NCELL);
+      const bool live = sq > 0.0;
+      scale = live ? sq : 0.0;
+      if (threadIdx.x == 0) P.scale[b] = scale;
+#pragma unroll
+      for (int k = 0; k < NV; ++k) {
+        const int c = threadIdx.x + k * FWD_THREADS;
+        const uint32_t lo = live ? f2bf((float)(rv[k] / sq)) : (uint16_t)0;
+        const uint32_t hi = f2bf((float)lv[k]);
+        F[((c >> 8) + 1) * FP + (((c >> 4) & 15) + 1) * HB + (c & 15) + 1] = lo | (hi << 16);
+        uint4* dst = reinterpret_cast<uint4*>(P.x0_out + ((size_t)b * NCELL + c) * CH);
+        dst[0] = make_uint4(lo | (hi << 16), 0u, 0u, 0u);
+        dst[1] = make_uint4(0u, 0u, 0u, 0u);
+      }
+      if (work + (int)gridDim.x < nwork) fetch(work + gridDim.x);
+    } else {
+      const int p0 = max(z0 - 3, 0), p1 = min(z0 + nz + 3, NB);
+      for (int c = p0 * 256 + threadIdx.x; c < p1 * 256; c += FWD_THREADS)
+        F[((c >> 8) + 1) * FP + (((c >> 4) & 15) + 1) * HB + (c & 15) + 1] =
+            *reinterpret_cast<const uint32_t*>(P.x0 + ((size_t)b * NCELL + c) * CH);
+    }
+    lds_barrier();
+
+    for (int i = z0 - 4; i < zend + 3; ++i) {
+      // layer 1, plane i + 2
+      if (i + 2 >= z0 - 2 && i + 2 < zend + 2) {
+        const int z = i + 2;
+        uint16_t* dst = h1 + (z & 3) * FWD_H * 8;
+        f32x4 acc[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
+        const bool in = (unsigned)z < (unsigned)NB;  // planes beyond the block are 0
+        if (in) {
+          const uint32_t* src = F + z * FP;
+#pragma unroll
+          for (int m = 0; m < 2; ++m)
+#pragma unroll
+            for (int q = 0; q < 2; ++q) {
+              const uint4 v = make_uint4(src[off1[m][0] + q * HB], src[off1[m][1] + q * HB],
+                                         src[off1[m][2] + q * HB], src[off1[m][3] + q * HB]);
+              acc[q] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, v),
+                                                               w1[m], acc[q], 0, 0, 0);
+            }
+        }
+#pragma unroll
+        for (int q = 0; q < 2; ++q)
+#pragma unroll
+          for (int j = 0; j < 4; ++j) {
+            const float v = acc[q][j] + b1;
+            dst[((y0 + q + 1) * HB + 4 * g + j + 1) * CH + cx] = f2bf(in && v > 0.f ? v : 0.f);
+          }
+      }
+      // layer 3, tap products of plane i - 2
+      if (i - 2 >= z0 && i - 2 < zend) {
+        float* dst = G + (i & 1) * FWD_G;
+#pragma unroll
+        for (int q = 0; q < 2; ++q) {
+          f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+          for (int m = 0; m < 2; ++m) {
+            const int dz = m == 0 ? tsel : 2;
+            acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+                __builtin_bit_cast(bf16x8, H2[((i - 3 + dz) & 3) * FWD_H +
+                                              ((y0 + q + 1) * HB + cx + 1) * 2 + half]),
+                w3[m], acc, 0, 0, 0);
+          }
+          if (cx < 9)
+#pragma unroll
+            for (int j = 0; j < 4; ++j) dst[((y0 + q + 1) * HB + 4 * g + j + 1) * 9 + cx] = acc[j];
+        }
+      }
+      // layer 2, plane i
+      if (i >= z0 - 1 && i < zend + 1) {
+        uint16_t* dst = h2 + (i & 3) * FWD_H * 8;
+        f32x4 acc[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
+        const bool in = (unsigned)i < (unsigned)NB;
+        if (in) {
+#pragma unroll
+          for (int rr = 0; rr < 4; ++rr) {  // input row y0 - 1 + rr, at padded y0 + rr
+            bf16x8 a[5];
+#pragma unroll
+            for (int f = 0; f < 5; ++f) {
+              const int dz = f < 3 ? f : (f == 3 ? tsel : 2), dx = f < 3 ? tsel : 2;
+              a[f] = __builtin_bit_cast(
+                  bf16x8, H1[((i + dz - 1) & 3) * FWD_H + ((y0 + rr) * HB + cx + dx) * 2 + half]);
+            }
+#pragma unroll
+            for (int f = 0; f < 5; ++f)
+#pragma unroll
+              for (int q = 0; q < 2; ++q) {
+                const int dy = rr - q;  // offset + 1 of output row y0 + q
+                if (dy >= 0 && dy < 3)
+                  acc[q] =
+                      __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[f], w2[f][dy], acc[q], 0, 0, 0);
+              }
+          }
+        }
+#pragma unroll
+        for (int q = 0; q < 2; ++q)
+#pragma unroll
+          for (int j = 0; j < 4; ++j) {
+            const float v = acc[q][j] + b2;
+            dst[((y0 + q + 1) * HB + 4 * g + j + 1) * CH + cx] = f2bf(in && v > 0.f ? v : 0.f);
+          }
+      }
+      // prediction of plane i - 3
+      if (i - 3 >= z0 && threadIdx.x < 256) {
+        const float* src = G + ((i - 1) & 1) * FWD_G;
+        const int x = threadIdx.x & 15, y = threadIdx.x >> 4;
+        float p = b3;
+#pragma unroll
+        for (int t = 0; t < 9; ++t) p += src[((y + t / 3) * HB + x + t % 3) * 9 + t];
+        const size_t c = (size_t)b * NCELL + (i - 3) * 256 + threadIdx.x;
+        P.pred[c] = p;
+        if (FROM_R) P.e[c] = P.omega * scale * (double)p;
+      }
+      // hidden planes to memory: the first layer's plane i + 1, the second's i - 1
+      if (SAVE) {
+        const int c = threadIdx.x >> 1, hf = threadIdx.x & 1;
+        const int at = (((c >> 4) + 1) * HB + (c & 15) + 1) * 2 + hf;
+        const int za = i + 1, zb = i - 1;
+        if (za >= z0 && za < zend)
+          reinterpret_cast<uint4*>(P.act[0])[((size_t)b * NCELL + za * 256 + c) * 2 + hf] =
+              H1[(za & 3) * FWD_H + at];
+        if (zb >= z0 && zb < zend)
+          reinterpret_cast<uint4*>(P.act[1])[((size_t)b * NCELL + zb * 256 + c) * 2 + hf] =
+              H2[(zb & 3) * FWD_H + at];
+      }
+      lds_barrier();
     }
   }
 }
@@ -650,6 +935,7 @@ struct Net {
   float* loss_partial = nullptr;
   float* loss = nullptr;
   double* blk[3] = {};         // level gathers: residual, log D, correction
+  int* unsaved = nullptr;      // blocks of the last pass whose act[1..2] were not stored
   int step = 0;
   int attached = 0;            // solvers using the network (learned_attach)
   int cin[NLAYER] = {2, CH, CH};
@@ -748,10 +1034,62 @@ void launch_wgrad(const uint16_t* x, const uint16_t* gz, float* partial, float* 
   hipLaunchKernelGGL(k_wgrad_reduce, dim3((GSZ + 15) / 16), dim3(256), 0, s, partial, nw, grad);
 }
 
+// Work-groups of k_forward: one per compute unit (its LDS allows no more).
+constexpr int kForwardGroups = 256;
+
+Forward forward_args(Net* n, int nblocks) {
+  Forward P{};
+  P.x0 = n->act[0];
+  P.x0_out = n->act[0];
+  P.scale = n->scale;
+  for (int l = 0; l < NLAYER; ++l) {
+    P.w[l] = n->wf[l];
+    P.bias[l] = n->bias[l];
+  }
+  P.act[0] = n->act[1];
+  P.act[1] = n->act[2];
+  P.pred = n->pred;
+  P.nblocks = nblocks;
+  P.unsaved = n->unsaved;
+  return P;
+}
+
+// Prediction and hidden activations from the features in act[0].  Work-groups
+// per block: whole blocks once they fill the compute units, else quarters
+// (which form five more planes of each layer than they need alone).
 void forward(Net* n, int nblocks, hipStream_t s) {
-  launch_conv(MODE_HIDDEN, n->act[0], n->wf[0], n->bias[0], nullptr, n->act[1], nullptr, nblocks, s);
-  launch_conv(MODE_HIDDEN, n->act[1], n->wf[1], n->bias[1], nullptr, n->act[2], nullptr, nblocks, s);
-  launch_conv(MODE_FINAL, n->act[2], n->wf[2], n->bias[2], nullptr, nullptr, n->pred, nblocks, s);
+  const int slabs = nblocks >= 256 ? 1 : 4;
+  hipLaunchKernelGGL((k_forward<true, false>), dim3(std::min(nblocks * slabs, kForwardGroups)),
+                     dim3(FWD_THREADS), 0, s, forward_args(n, nblocks), slabs);
+}
+
+// Scale, features, prediction and correction e of every block from r and
+// log D.  The hidden activations, which only a backward pass reads, are not
+// stored; *unsaved says so on the device, so that a replayed graph of this
+// call says so too.
+void correction(Net* n, const double* r, const double* logd, double logd_const, double h2,
+                double omega, double* e, int nblocks, hipStream_t s) {
+  Forward P = forward_args(n, nblocks);
+  P.r = r;
+  P.logd = logd;
+  P.logd_const = logd_const;
+  P.h2 = h2;
+  P.omega = omega;
+  P.e = e;
+  hipLaunchKernelGGL((k_forward<false, true>), dim3(std::min(nblocks, kForwardGroups)),
+                     dim3(FWD_THREADS), 0, s, P, 1);
+}
+
+__global__ void k_set_int(int* p, int v) { *p = v; }
+
+// The hidden activations a correction left out, before anything that reads
+// them or changes the weights they come from.
+void save_hidden(Net* n, hipStream_t s) {
+  Forward P = forward_args(n, n->max_blocks);
+  P.only_unsaved = 1;
+  hipLaunchKernelGGL((k_forward<true, false>), dim3(std::min(n->max_blocks, kForwardGroups)),
+                     dim3(FWD_THREADS), 0, s, P, 1);
+  hipLaunchKernelGGL(k_set_int, dim3(1), dim3(1), 0, s, n->unsaved, 0);
 }
 
 // Loss and gradients of every layer (after forward on the same features).
@@ -824,6 +1162,7 @@ void free_net(Net* n) {
   (void)hipFree(n->partial);
   (void)hipFree(n->loss_partial);
   (void)hipFree(n->loss);
+  (void)hipFree(n->unsaved);
   for (int k = 0; k < 3; ++k) (void)hipFree(n->blk[k]);
   delete n;
 }
@@ -879,11 +1218,7 @@ int learned_correct_level(void* net, double* const* utab, int ughost, double* co
                          nblocks, n->blk[1]);
       logd = n->blk[1];
     }
-    hipLaunchKernelGGL(k_features, dim3(nblocks), dim3(256), 0, s, n->blk[0], logd, logd_const, h * h,
-                       n->act[0], n->scale);
-    forward(n, nblocks, s);
-    hipLaunchKernelGGL(k_correction, grid, block, 0, s, n->pred, n->scale, omega, ncells,
-                       n->blk[2]);
+    correction(n, n->blk[0], logd, logd_const, h * h, omega, n->blk[2], nblocks, s);
     hipLaunchKernelGGL(k_add_blocks, grid, block, 0, s, utab, ughost, windows, nblocks,
                        n->blk[2]);
   });
@@ -1000,6 +1335,8 @@ int sfac_learned_create(int max_blocks, unsigned long long seed, void** out) {
       n->partial = dalloc<float>((size_t)wgrad_waves(max_blocks * NROW) * GSZ);
       n->loss_partial = dalloc<float>((ncells + 255) / 256);
       n->loss = dalloc<float>(1);
+      n->unsaved = dalloc<int>(1);
+      ck(hipMemset(n->unsaved, 0, sizeof(int)));
       for (int k = 0; k < 3; ++k) n->blk[k] = dalloc<double>(ncells);
       init_params(n, seed, 0);
       ck(hipStreamSynchronize(0));
@@ -1054,11 +1391,23 @@ int sfac_learned_correction(void* net, double omega, double* e, int nblocks, hip
   });
 }
 
+int sfac_learned_apply(void* net, const double* r, const double* logd, double h, double omega,
+                       double* e, int nblocks, hipStream_t stream) {
+  return guarded([&] {
+    Net* n = net_of(net, nblocks);
+    need(r && e, "null residual or correction");
+    need(h > 0.0, "h must be positive");
+    if (nblocks == 0) return;
+    correction(n, r, logd, 0.0, h * h, omega, e, nblocks, stream);
+  });
+}
+
 int sfac_learned_backward(void* net, const double* target, int nblocks, hipStream_t stream) {
   return guarded([&] {
     Net* n = net_of(net, nblocks);
     need(target != nullptr, "null target");
     need(nblocks > 0, "backward needs at least one block");
+    save_hidden(n, stream);
     backward(n, target, nblocks, stream);
   });
 }
@@ -1066,6 +1415,7 @@ int sfac_learned_backward(void* net, const double* target, int nblocks, hipStrea
 int sfac_learned_adam(void* net, float lr, hipStream_t stream) {
   return guarded([&] {
     Net* n = net_of(net, 0);
+    save_hidden(n, stream);
     const float b1 = 0.9f, b2 = 0.999f, eps = 1e-8f;
     n->step += 1;
     const float bc1 = 1.f - std::pow(b1, (float)n->step);
@@ -1117,6 +1467,7 @@ int sfac_learned_set_params(void* net, const float* host) {
   return guarded([&] {
     Net* n = net_of(net, 0);
     need(host != nullptr, "null host buffer");
+    save_hidden(n, 0);
     for (int l = 0; l < NLAYER; ++l) {
       ck(hipMemcpy(n->p[l], host + (size_t)l * PSZ, PSZ * sizeof(float), hipMemcpyHostToDevice));
       ck(hipMemset(n->m[l], 0, PSZ * sizeof(float)));

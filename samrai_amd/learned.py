@@ -50,6 +50,7 @@ def lib():
     L.sfac_learned_features.argtypes = [_vp, _vp, _vp, d, i, _vp]
     L.sfac_learned_forward.argtypes = [_vp, i, _vp]
     L.sfac_learned_correction.argtypes = [_vp, d, _vp, i, _vp]
+    L.sfac_learned_apply.argtypes = [_vp, _vp, _vp, d, d, _vp, i, _vp]
     L.sfac_learned_backward.argtypes = [_vp, _vp, i, _vp]
     L.sfac_learned_adam.argtypes = [_vp, f, _vp]
     L.sfac_learned_train_step.argtypes = [_vp, _vp, _vp, _vp, d, i, f, _vp]
@@ -194,10 +195,10 @@ class LearnedSmoother:
 
     def correction(self, r, logd, h, omega=1.0):
         """e = omega * s * net(r h^2 / s, log D), FP64 per cell."""
-        n = self.forward(r, logd, h)
+        n = self._n(r)
         e = self.torch.empty_like(r)
-        fac._check(lib().sfac_learned_correction(self.h, float(omega), _p(e), n,
-                                                 _stream(self.torch)))
+        fac._check(lib().sfac_learned_apply(self.h, _p(r), _p(logd), float(h), float(omega),
+                                            _p(e), n, _stream(self.torch)))
         return e
 
     def backward(self, target):

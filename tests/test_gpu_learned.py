@@ -199,6 +199,57 @@ def test_block_sor_from_a_start_matches_oracle(torch_gpu, blocks, sweeps, omega,
     assert np.abs(e - eo).max() <= 64 * 2.0 ** -52 * max(1, sweeps) * top
 
 
+@pytest.mark.parametrize("blocks", [1, 63, 256, 300])
+def test_backward_after_a_correction_equals_backward_after_forward(torch_gpu, blocks):
+    """A correction does not store the hidden activations, a forward pass
+    does: a backward pass (and an optimizer step and new weights) after either
+    sees the same network, and the features, predictions and scales are the same.  Block counts below and above the compute units, where a
+    work-group takes a quarter of a block, a block, and several."""
+    torch = torch_gpu
+    from samrai_amd import learned as SL
+    _say("backward after a correction, %d blocks" % blocks)
+    g = torch.Generator(device="cuda").manual_seed(blocks)
+    r, logd, t = (torch.randn((blocks, 16, 16, 16), generator=g, dtype=torch.float64,
+                              device="cuda") for _ in range(3))
+    r[blocks // 2] = 0.0  # a block without a residual
+    out = []
+    for use_correction in (False, True):
+        net = SL.LearnedSmoother(torch, blocks, seed=3)
+        h = 1.0 / 32
+        if use_correction:
+            e = net.correction(r, logd, h, 0.7)
+        else:
+            net.forward(r, logd, h)
+            e = torch.empty_like(r)
+            SL.fac._check(SL.lib().sfac_learned_correction(net.h, 0.7, SL._p(e), blocks,
+                                                           SL._stream(torch)))
+        feat, pred, scale = net.buffers()
+        got = [e.cpu().numpy(), _wrap(torch, feat, blocks * 4096 * 16, torch.int16).cpu().numpy(),
+               _wrap(torch, pred, blocks * 4096, torch.float32).cpu().numpy(),
+               _wrap(torch, scale, blocks, torch.float64).cpu().numpy()]
+        net.backward(t)
+        got += net.grads() + [np.float32(net.loss())]
+        SL.fac._check(SL.lib().sfac_learned_adam(net.h, 1e-3, SL._stream(torch)))
+        got += net.params()
+        out.append(got)
+        net.close()
+    # the scales sum 4096 squares in another order; a block with the same scale
+    # has the same bits throughout
+    ref, cor = out
+    np.testing.assert_allclose(cor[3], ref[3], rtol=4096 * 2.0 ** -53)
+    same = cor[3] == ref[3]
+    assert same.sum() >= blocks // 2
+    for k in range(3):
+        a, b = (v[k].reshape(blocks, -1)[same] for v in (ref, cor))
+        np.testing.assert_array_equal(a, b)
+    # sums over all blocks: a flipped BF16 rounding of a feature (2^-9 of it)
+    # in the others; the first Adam step moves a weight by at most lr
+    for k in range(4, 8):
+        assert np.linalg.norm(cor[k] - ref[k]) <= 1e-3 * np.linalg.norm(ref[k])
+    for k in range(8, 11):
+        assert np.abs(cor[k] - ref[k]).max() <= 2.1e-3
+
+
 def test_training_on_fac_pairs_gains_over_no_network(torch_gpu):
     torch = torch_gpu
     from samrai_amd import learned as SL
