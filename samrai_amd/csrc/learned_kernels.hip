@@ -13,8 +13,8 @@
 // convolution accumulates in FP32.  Channel counts are padded to 16 so that
 // every layer is the same implicit GEMM: per output row of 16 cells and per
 // pair of taps, one v_mfma_f32_16x16x32_bf16 with M = 16 cells, N = 16
-// output channels, K = 2 taps x 16 input channels (the weight gradient uses
-// v_mfma_f32_16x16x16_bf16 with K = 16 cells).
+// output channels, K = 2 taps x 16 input channels (the weight gradient has
+// K = 32 cells).
 //
 // Activations are channels-last BF16: act[block][z][y][x][16] (32 B per
 // cell).  Convolution weights are stored per tap: wf[t][co][ci] (forward)
@@ -40,16 +40,13 @@ namespace {
 
 constexpr int NB = 16;                 // block side
 constexpr int NCELL = NB * NB * NB;    // cells per block
-constexpr int NROW = NB * NB;          // 16-cell rows per block
 constexpr int CH = 16;                 // padded channel count
 constexpr int NTAP = 27;
 constexpr int WSZ = NTAP * CH * CH;    // conv weights per layer
 constexpr int PSZ = WSZ + CH;          // + bias
 constexpr int GSZ = (NTAP + 1) * CH * CH;  // gradient slab: 27 taps + bias row
 constexpr int NLAYER = 3;
-constexpr int WGRAD_ROWS = 16;         // rows accumulated per wave in the weight gradient
 
-typedef short bf16x4 __attribute__((ext_vector_type(4)));
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 constexpr int NPAIR = (NTAP + 1) / 2;  // tap pairs per K = 32 MFMA
 typedef float f32x4 __attribute__((ext_vector_type(4)));
@@ -70,17 +67,6 @@ __host__ __device__ inline float bf2f(uint16_t h) {
   float f;
   memcpy(&f, &u, 4);
   return f;
-}
-
-__device__ inline bf16x4 load4(const uint16_t* p) {
-  // 8-byte aligned: channel groups start at multiples of 4
-  uint2 v = *reinterpret_cast<const uint2*>(p);
-  bf16x4 r;
-  r[0] = (short)(v.x & 0xffffu);
-  r[1] = (short)(v.x >> 16);
-  r[2] = (short)(v.y & 0xffffu);
-  r[3] = (short)(v.y >> 16);
-  return r;
 }
 
 enum { MODE_HIDDEN = 0, MODE_FINAL = 1, MODE_BWD = 2 };
@@ -454,128 +440,219 @@ __global__ __launch_bounds__(FWD_THREADS) void k_forward(Forward P, int slabs) {
 }
 
 // Weight gradient: dW[t][co][ci] = sum_cells G[cell][co] X[cell + off(t)][ci],
-// db[co] = sum_cells G[cell][co].  Each wave accumulates WGRAD_ROWS rows into
-// 28 MFMA tiles (27 taps + the bias row, whose B operand is 1 in column 0)
-// and writes its partial slab; k_wgrad_reduce sums the slabs in a fixed order.
-// A[m][k] (lane l: m = co = l & 15, k = cells 4g..4g+3) = G[cell_k][co]
-// B[k][n] (lane l: n = ci = l & 15, k = cells 4g..4g+3) = X[cell_k + off(t)][ci]
+// db[co] = sum_cells G[cell][co]: 28 products per 32 cells (27 taps and a ones
+// column), K = 32 cells = two rows of 16.  Both operands need a channel's cells
+// consecutive while memory holds a cell's channels so, and read from memory
+// they are 2-byte loads, which bound the first version (69 us for 64 blocks).
+// Here a work-group stages the planes of its z-slab once, transposed in LDS
+// ([channel][row][cell], rows of 24 elements whose first 8 are zeros: 16-byte
+// reads of eight cells, the neighbouring row's zeros at both ends), a ring of
+// four planes of X and two of G so that the next planes load and store while
+// the current ones are multiplied; a (dz, dy) row is read once and its dx = -1
+// and 1 neighbours are formed by 32-bit funnel shifts.  The channel strides
+// (220 and 132 words) spread 16 channels over all LDS banks.  A training
+// step of 64 blocks (three of these, the rest of the network and Adam) 0.37 ms
+// with the first version, 0.12 ms with this one and the fused forward pass.
+// A[m][k] (lane l: m = co = l & 15, k = cells 8g..8g+7) = G[cell_k][co]
+// B[k][n] (lane l: n = ci = l & 15, k = cells 8g..8g+7) = X[cell_k + off(t)][ci]
 // D[m][n] (lane l: m = 4g + j, n = l & 15) -> partial[t][m][n]
+constexpr int WG_ROW = 24;                  // elements of a staged row of X
+constexpr int WG_XC = 440;                  // per channel: 18 rows and padding
+constexpr int WG_XP = CH * WG_XC;           // per plane
+constexpr int WG_GC = 264;                  // per channel of G: 256 cells and padding
+constexpr int WG_GP = CH * WG_GC;
+constexpr int WG_LDS = 4 * WG_XP + 2 * WG_GP;  // 73,216 B: two work-groups a CU
+
 __global__ __launch_bounds__(256) void k_wgrad(const uint16_t* __restrict__ x,
                                                const uint16_t* __restrict__ gz,
-                                               float* __restrict__ partial, int nrows,
-                                               int nwaves) {
-  const int lane = threadIdx.x & 63;
-  const int wave = blockIdx.x * 4 + (threadIdx.x >> 6);
-  if (wave >= nwaves) return;
-  const int cx = lane & 15;
-  const int g = lane >> 4;
+                                               float* __restrict__ partial, int nblocks,
+                                               int slabs) {
+  __shared__ __align__(16) uint16_t lds[WG_LDS];
+  uint16_t* X = lds;
+  uint16_t* Gs = lds + 4 * WG_XP;
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int cx = lane & 15, g = lane >> 4;
+  const int tx = threadIdx.x & 15, ty = threadIdx.x >> 4;  // staged cell
+  const int nz = NB / slabs, nwork = nblocks * slabs;
+  for (int q = threadIdx.x; q < WG_LDS / 8; q += 256)
+    reinterpret_cast<uint4*>(lds)[q] = make_uint4(0u, 0u, 0u, 0u);
   f32x4 acc[NTAP + 1];
 #pragma unroll
   for (int t = 0; t <= NTAP; ++t) acc[t] = f32x4{0.f, 0.f, 0.f, 0.f};
-  bf16x4 ones;
+  bf16x8 ones;
   {
-    const short one = (short)f2bf(1.0f);
-    const short v = cx == 0 ? one : (short)0;
-    ones = bf16x4{v, v, v, v};
+    const uint32_t v = cx == 0 ? 0x3f803f80u : 0u;
+    ones = __builtin_bit_cast(bf16x8, make_uint4(v, v, v, v));
   }
-  const int r0 = wave * WGRAD_ROWS;
-  const int r1 = min(nrows, r0 + WGRAD_ROWS);
-  for (int row = r0; row < r1; ++row) {
-    const int b = row / NROW;
-    const int y = row % NB;
-    const int z = (row / NB) % NB;
-    const uint16_t* xb = x + (size_t)b * NCELL * CH;
-    const size_t cell0 = (size_t)row * NB;
-    bf16x4 a;
-#pragma unroll
-    for (int j = 0; j < 4; ++j) a[j] = (short)gz[(cell0 + 4 * g + j) * CH + cx];
-    // per (dz, dy): the six cells x = 4g-1 .. 4g+4 of channel ci serve all three dx taps
-#pragma unroll
-    for (int q = 0; q < 9; ++q) {
-      const int dz = q / 3 - 1, dy = q % 3 - 1;
-      const int yy = y + dy, zz = z + dz;
-      short v[6] = {0, 0, 0, 0, 0, 0};
-      if ((unsigned)yy < (unsigned)NB && (unsigned)zz < (unsigned)NB) {
-        const uint16_t* xr = xb + (size_t)((zz * NB + yy) * NB) * CH + cx;
-#pragma unroll
-        for (int k = 0; k < 6; ++k) {
-          const int xx = 4 * g - 1 + k;
-          if ((unsigned)xx < (unsigned)NB) v[k] = (short)xr[xx * CH];
-        }
-      }
-#pragma unroll
-      for (int dx = -1; dx <= 1; ++dx) {
-        const bf16x4 bx = {v[1 + dx], v[2 + dx], v[3 + dx], v[4 + dx]};
-        const int t = 3 * q + dx + 1;
-        acc[t] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a, bx, acc[t], 0, 0, 0);
-      }
+  struct Cell {
+    uint4 lo, hi;
+  };
+  auto load = [&](const uint16_t* p, int b, int z) {  // plane z's cell of this thread
+    Cell c{make_uint4(0u, 0u, 0u, 0u), make_uint4(0u, 0u, 0u, 0u)};
+    if ((unsigned)z < (unsigned)NB) {
+      const uint4* q =
+          reinterpret_cast<const uint4*>(p + ((size_t)b * NCELL + z * 256 + threadIdx.x) * CH);
+      c.lo = q[0];
+      c.hi = q[1];
     }
-    acc[NTAP] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a, ones, acc[NTAP], 0, 0, 0);
+    return c;
+  };
+  auto store = [&](uint16_t* dst, int stride, const Cell& c) {  // a channel per `stride`
+    const uint32_t w[8] = {c.lo.x, c.lo.y, c.lo.z, c.lo.w, c.hi.x, c.hi.y, c.hi.z, c.hi.w};
+#pragma unroll
+    for (int k = 0; k < 8; ++k) {
+      dst[(2 * k) * stride] = (uint16_t)(w[k] & 0xffffu);
+      dst[(2 * k + 1) * stride] = (uint16_t)(w[k] >> 16);
+    }
+  };
+  auto xcell = [&](int z) { return X + ((z + 4) & 3) * WG_XP + (ty + 1) * WG_ROW + 8 + tx; };
+  auto gcell = [&](int z) { return Gs + (z & 1) * WG_GP + threadIdx.x; };
+  lds_barrier();
+  for (int work = blockIdx.x; work < nwork; work += gridDim.x) {
+    const int b = work / slabs, z0 = (work % slabs) * nz;
+    {
+      const Cell a0 = load(x, b, z0 - 1), a1 = load(x, b, z0), a2 = load(x, b, z0 + 1);
+      const Cell g0 = load(gz, b, z0);
+      store(xcell(z0 - 1), WG_XC, a0);
+      store(xcell(z0), WG_XC, a1);
+      store(xcell(z0 + 1), WG_XC, a2);
+      store(gcell(z0), WG_GC, g0);
+    }
+    lds_barrier();
+    for (int z = z0; z < z0 + nz; ++z) {
+      const bool more = z + 1 < z0 + nz;
+      Cell xn{}, gn{};
+      if (more) {
+        xn = load(x, b, z + 2);
+        gn = load(gz, b, z + 1);
+      }
+#pragma unroll
+      for (int rp = 0; rp < 2; ++rp) {
+        const int y = 2 * (wave + 4 * rp) + (g >> 1), xo = 8 * (g & 1);
+        const bf16x8 a = __builtin_bit_cast(
+            bf16x8, *reinterpret_cast<const uint4*>(Gs + (z & 1) * WG_GP + cx * WG_GC + 16 * y + xo));
+#pragma unroll
+        for (int q = 0; q < 9; ++q) {
+          const int dz = q / 3 - 1, dy = q % 3 - 1;
+          const uint16_t* row =
+              X + ((z + dz + 4) & 3) * WG_XP + cx * WG_XC + (y + dy + 1) * WG_ROW + 8 + xo;
+          const uint4 v = *reinterpret_cast<const uint4*>(row);
+          const uint32_t lo = row[-1], hi = row[8];
+          // eight cells from x - 1 and from x + 1
+          const uint32_t s0 = __builtin_amdgcn_alignbit(v.x, lo << 16, 16);
+          const uint32_t s1 = __builtin_amdgcn_alignbit(v.y, v.x, 16);
+          const uint32_t s2 = __builtin_amdgcn_alignbit(v.z, v.y, 16);
+          const uint32_t s3 = __builtin_amdgcn_alignbit(v.w, v.z, 16);
+          const uint32_t s4 = __builtin_amdgcn_alignbit(hi, v.w, 16);
+          acc[3 * q] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+              a, __builtin_bit_cast(bf16x8, make_uint4(s0, s1, s2, s3)), acc[3 * q], 0, 0, 0);
+          acc[3 * q + 1] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+              a, __builtin_bit_cast(bf16x8, v), acc[3 * q + 1], 0, 0, 0);
+          acc[3 * q + 2] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+              a, __builtin_bit_cast(bf16x8, make_uint4(s1, s2, s3, s4)), acc[3 * q + 2], 0, 0, 0);
+        }
+        acc[NTAP] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, ones, acc[NTAP], 0, 0, 0);
+      }
+      if (more) {  // planes z + 2 and z + 1: slots the current step does not read
+        store(xcell(z + 2), WG_XC, xn);
+        store(gcell(z + 1), WG_GC, gn);
+      }
+      lds_barrier();
+    }
   }
-  float* p = partial + (size_t)wave * GSZ;
+  // the four wavefronts' sums, in a fixed order, into one slab
+  float* red = reinterpret_cast<float*>(lds);  // two slabs of GSZ floats
+  auto put = [&](float* p) {
 #pragma unroll
-  for (int t = 0; t <= NTAP; ++t)
+    for (int t = 0; t <= NTAP; ++t)
 #pragma unroll
-    for (int j = 0; j < 4; ++j) p[(t * CH + 4 * g + j) * CH + cx] = acc[t][j];
+      for (int j = 0; j < 4; ++j) p[(t * CH + 4 * g + j) * CH + cx] = acc[t][j];
+  };
+  auto add = [&](const float* p) {
+#pragma unroll
+    for (int t = 0; t <= NTAP; ++t)
+#pragma unroll
+      for (int j = 0; j < 4; ++j) acc[t][j] += p[(t * CH + 4 * g + j) * CH + cx];
+  };
+  static_assert(2 * GSZ * 4 <= WG_LDS * 2, "two slabs fit the staging buffer");
+  if (wave >= 2) put(red + (wave - 2) * GSZ);
+  __syncthreads();
+  if (wave < 2) add(red + wave * GSZ);
+  __syncthreads();
+  if (wave == 1) put(red);
+  __syncthreads();
+  if (wave == 0) {
+    add(red);
+    put(partial + (size_t)blockIdx.x * GSZ);
+  }
 }
 
-// Sum of the per-wave slabs: a work-group per 16 outputs, 16 threads per
-// output each summing every 16th slab in order, then the 16 partial sums in
-// a fixed order (deterministic).
+// Sum of the work-groups' slabs: 16 threads per output each summing every
+// 16th slab in order, then the 16 partial sums in a fixed order
+// (deterministic).  blockIdx.y: a layer, `layer_stride` slabs apart.
+struct GradOut {
+  float* grad[NLAYER];
+};
 __global__ __launch_bounds__(256) void k_wgrad_reduce(const float* __restrict__ partial,
-                                                      int nwaves, float* __restrict__ grad) {
+                                                      int nslabs, size_t layer_stride,
+                                                      GradOut out) {
   __shared__ float red[16][17];
   const int o = threadIdx.x & 15;
   const int part = threadIdx.x >> 4;
   const int i = blockIdx.x * 16 + o;
+  const float* p = partial + blockIdx.y * layer_stride;
   float s = 0.f;
   if (i < GSZ)
-    for (int w = part; w < nwaves; w += 16) s += partial[(size_t)w * GSZ + i];
+    for (int w = part; w < nslabs; w += 16) s += p[(size_t)w * GSZ + i];
   red[part][o] = s;
   __syncthreads();
   if (part == 0 && i < GSZ) {
     float t = 0.f;
 #pragma unroll
     for (int k = 0; k < 16; ++k) t += red[k][o];
-    grad[i] = t;
+    out.grad[blockIdx.y][i] = t;
   }
 }
 
-// Features of one block per work-group (256 threads, 16 cells each):
-// s = RMS over the block of r h^2 (1 if zero); X[cell] = (r h^2 / s, log D, 0...).
-__global__ __launch_bounds__(256) void k_features(const double* __restrict__ r,
-                                                  const double* __restrict__ logd,
-                                                  double logd_const, double h2,
-                                                  uint16_t* __restrict__ x,
-                                                  double* __restrict__ scale) {
-  __shared__ double red[256];
+// Features of one block per work-group (1024 threads, four cells each, read
+// once: a training batch has fewer blocks than there are compute units, and its
+// time is this chain's): s = RMS over the block of r h^2;
+// X[cell] = (r h^2 / s, log D, 0...).
+constexpr int kFeatThreads = 1024;
+__global__ __launch_bounds__(kFeatThreads) void k_features(const double* __restrict__ r,
+                                                           const double* __restrict__ logd,
+                                                           double logd_const, double h2,
+                                                           uint16_t* __restrict__ x,
+                                                           double* __restrict__ scale) {
+  constexpr int NV = NCELL / kFeatThreads;
+  __shared__ double red[kFeatThreads / 64];
   const int b = blockIdx.x;
-  const double* rb = r + (size_t)b * NCELL;
-  double s2 = 0.0;
-  for (int c = threadIdx.x; c < NCELL; c += 256) {
-    const double v = rb[c] * h2;
-    s2 += v * v;
+  const size_t c0 = (size_t)b * NCELL + threadIdx.x;
+  double v[NV], l[NV], s2 = 0.0;
+#pragma unroll
+  for (int k = 0; k < NV; ++k) {
+    v[k] = r[c0 + k * kFeatThreads] * h2;
+    l[k] = logd ? logd[c0 + k * kFeatThreads] : logd_const;
   }
-  red[threadIdx.x] = s2;
+#pragma unroll
+  for (int k = 0; k < NV; ++k) s2 += v[k] * v[k];
+  for (int o = 32; o > 0; o >>= 1) s2 += __shfl_xor(s2, o, 64);
+  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = s2;
   __syncthreads();
-  for (int k = 128; k > 0; k >>= 1) {
-    if ((int)threadIdx.x < k) red[threadIdx.x] += red[threadIdx.x + k];
-    __syncthreads();
-  }
+  s2 = 0.0;
+#pragma unroll
+  for (int k = 0; k < kFeatThreads / 64; ++k) s2 += red[k];
   // a block whose residual is zero (or not finite) gets scale 0: zero
   // features, a zero correction and no loss term
-  const double s = sqrt(red[0] / NCELL);
+  const double s = sqrt(s2 / NCELL);
   const bool live = s > 0.0;
   if (threadIdx.x == 0) scale[b] = live ? s : 0.0;
-  uint16_t* xb = x + (size_t)b * NCELL * CH;
-  for (int c = threadIdx.x; c < NCELL; c += 256) {
-    uint16_t v[CH];
 #pragma unroll
-    for (int k = 0; k < CH; ++k) v[k] = 0;
-    v[0] = live ? f2bf((float)(rb[c] * h2 / s)) : (uint16_t)0;
-    v[1] = f2bf((float)(logd ? logd[(size_t)b * NCELL + c] : logd_const));
-    uint4* dst = reinterpret_cast<uint4*>(xb + (size_t)c * CH);
-    dst[0] = make_uint4(v[0] | (v[1] << 16), 0u, 0u, 0u);
+  for (int k = 0; k < NV; ++k) {
+    const uint32_t lo = live ? f2bf((float)(v[k] / s)) : (uint16_t)0;
+    const uint32_t hi = f2bf((float)l[k]);
+    uint4* dst = reinterpret_cast<uint4*>(x + (c0 + k * kFeatThreads) * CH);
+    dst[0] = make_uint4(lo | (hi << 16), 0u, 0u, 0u);
     dst[1] = make_uint4(0u, 0u, 0u, 0u);
   }
 }
@@ -621,14 +698,22 @@ __global__ void k_sum_f32(const float* __restrict__ a, int n, float scale_by,
   if (threadIdx.x == 0) out[0] = red[0] * scale_by;
 }
 
-// Adam on the FP32 master parameters of one layer (27*16*16 weights then 16
-// biases), then the BF16 copies in forward and (flipped, transposed)
+// Adam on the FP32 master parameters of layer blockIdx.y (27*16*16 weights
+// then 16 biases), then the BF16 copies in forward and (flipped, transposed)
 // backward layouts.  Weights outside the layer's real channel counts stay 0.
-__global__ void k_adam(float* __restrict__ p, float* __restrict__ m, float* __restrict__ v,
-                       const float* __restrict__ grad, int cin, int cout, float lr,
-                       float beta1, float beta2, float eps, float bc1, float bc2,
-                       uint16_t* __restrict__ wf, uint16_t* __restrict__ wb,
-                       float* __restrict__ bias) {
+struct AdamLayer {
+  float *p, *m, *v;
+  const float* grad;
+  uint16_t *wf, *wb;
+  float* bias;
+  int cin, cout;
+};
+struct AdamLayers {
+  AdamLayer l[NLAYER];
+};
+__global__ void k_adam(AdamLayers all, float lr, float beta1, float beta2, float eps, float bc1,
+                       float bc2) {
+  const AdamLayer L = all.l[blockIdx.y];
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= PSZ) return;
   float gi;
@@ -638,30 +723,30 @@ __global__ void k_adam(float* __restrict__ p, float* __restrict__ m, float* __re
     t = i / (CH * CH);
     co = (i / CH) % CH;
     ci = i % CH;
-    live = ci < cin && co < cout;
-    gi = grad[i];
+    live = ci < L.cin && co < L.cout;
+    gi = L.grad[i];
   } else {
     co = i - WSZ;
-    live = co < cout;
-    gi = grad[(NTAP * CH + co) * CH + 0];
+    live = co < L.cout;
+    gi = L.grad[(NTAP * CH + co) * CH + 0];
   }
-  float pi = p[i];
+  float pi = L.p[i];
   if (live) {
-    const float mi = beta1 * m[i] + (1.f - beta1) * gi;
-    const float vi = beta2 * v[i] + (1.f - beta2) * gi * gi;
-    m[i] = mi;
-    v[i] = vi;
+    const float mi = beta1 * L.m[i] + (1.f - beta1) * gi;
+    const float vi = beta2 * L.v[i] + (1.f - beta2) * gi * gi;
+    L.m[i] = mi;
+    L.v[i] = vi;
     pi -= lr * (mi / bc1) / (sqrtf(vi / bc2) + eps);
   } else {
     pi = 0.f;
   }
-  p[i] = pi;
+  L.p[i] = pi;
   if (i < WSZ) {
     const uint16_t h = f2bf(pi);
-    wf[(t * CH + co) * CH + ci] = h;
-    wb[((NTAP - 1 - t) * CH + ci) * CH + co] = h;
+    L.wf[(t * CH + co) * CH + ci] = h;
+    L.wb[((NTAP - 1 - t) * CH + ci) * CH + co] = h;
   } else {
-    bias[co] = pi;
+    L.bias[co] = pi;
   }
 }
 
@@ -978,7 +1063,12 @@ T* dalloc(size_t n) {
   return static_cast<T*>(ptr);
 }
 
-int wgrad_waves(int nrows) { return (nrows + WGRAD_ROWS - 1) / WGRAD_ROWS; }
+// Work-groups (slabs of partial sums) of the weight gradient, and z-slabs per
+// block: quarters of a block while whole ones would leave compute units idle,
+// at most two work-groups per compute unit, which then take several.
+constexpr int kWgradGroups = 512;
+int wgrad_slabs(int nblocks) { return nblocks < 128 ? 4 : 1; }
+int wgrad_groups(int nblocks) { return std::min(nblocks * wgrad_slabs(nblocks), kWgradGroups); }
 
 // Per-wave gradient slabs of the allocation-free weight gradient
 // (sfac_conv3x3x3_wgrad_bf16_noalloc): one array per GPU, held until the
@@ -986,8 +1076,8 @@ int wgrad_waves(int nrows) { return (nrows + WGRAD_ROWS - 1) / WGRAD_ROWS; }
 // host it names a stand-in, not device memory): it passes the address that
 // hipGetSymbolAddress returns for the current device.
 constexpr int NOALLOC_MAX_BLOCKS = SFAC_WGRAD_NOALLOC_MAX_BLOCKS;
-constexpr size_t NOALLOC_FLOATS = (size_t)((NOALLOC_MAX_BLOCKS * NROW + WGRAD_ROWS - 1) /
-                                           WGRAD_ROWS) * GSZ;  // 7 MiB
+constexpr size_t NOALLOC_FLOATS = (size_t)NOALLOC_MAX_BLOCKS * 16 * GSZ;  // 7 MiB
+static_assert(NOALLOC_MAX_BLOCKS < 128, "four slabs a block, 16 fit");
 __device__ __align__(256) float scratch[NOALLOC_FLOATS];
 
 constexpr int kMaxDevices = 64;
@@ -1026,12 +1116,18 @@ void launch_conv(int mode, const uint16_t* x, const uint16_t* w, const float* bi
                        nplanes);
 }
 
+void launch_wgrad_partial(const uint16_t* x, const uint16_t* gz, float* partial, int nblocks,
+                          hipStream_t s) {
+  hipLaunchKernelGGL(k_wgrad, dim3(wgrad_groups(nblocks)), dim3(256), 0, s, x, gz, partial, nblocks,
+                     wgrad_slabs(nblocks));
+}
+
 void launch_wgrad(const uint16_t* x, const uint16_t* gz, float* partial, float* grad, int nblocks,
                   hipStream_t s) {
-  const int nrows = nblocks * NROW;
-  const int nw = wgrad_waves(nrows);
-  hipLaunchKernelGGL(k_wgrad, dim3((nw + 3) / 4), dim3(256), 0, s, x, gz, partial, nrows, nw);
-  hipLaunchKernelGGL(k_wgrad_reduce, dim3((GSZ + 15) / 16), dim3(256), 0, s, partial, nw, grad);
+  launch_wgrad_partial(x, gz, partial, nblocks, s);
+  GradOut out{{grad, nullptr, nullptr}};
+  hipLaunchKernelGGL(k_wgrad_reduce, dim3((GSZ + 15) / 16), dim3(256), 0, s, partial,
+                     wgrad_groups(nblocks), (size_t)0, out);
 }
 
 // Work-groups of k_forward: one per compute unit (its LDS allows no more).
@@ -1100,14 +1196,32 @@ void backward(Net* n, const double* target, int nblocks, hipStream_t s) {
                      1.f / (float)ncells, n->gbuf[0], n->loss_partial);
   hipLaunchKernelGGL(k_sum_f32, dim3(1), dim3(256), 0, s, n->loss_partial, nlb,
                      1.f / (float)ncells, n->loss);
-  // layer 3: gradient gbuf[0] (channel 0 only)
-  launch_wgrad(n->act[2], n->gbuf[0], n->partial, n->grad[2], nblocks, s);
+  // layer 3: gradient gbuf[0] (channel 0 only); the layers' partial sums side
+  // by side, summed in one launch
+  const size_t stride = (size_t)wgrad_groups(nblocks) * GSZ;
+  launch_wgrad_partial(n->act[2], n->gbuf[0], n->partial + 2 * stride, nblocks, s);
   launch_conv(MODE_BWD, n->gbuf[0], n->wb[2], nullptr, n->act[2], n->gbuf[1], nullptr, nblocks, s);
   // layer 2
-  launch_wgrad(n->act[1], n->gbuf[1], n->partial, n->grad[1], nblocks, s);
+  launch_wgrad_partial(n->act[1], n->gbuf[1], n->partial + stride, nblocks, s);
   launch_conv(MODE_BWD, n->gbuf[1], n->wb[1], nullptr, n->act[1], n->gbuf[0], nullptr, nblocks, s);
   // layer 1 (its input gradient is not needed)
-  launch_wgrad(n->act[0], n->gbuf[0], n->partial, n->grad[0], nblocks, s);
+  launch_wgrad_partial(n->act[0], n->gbuf[0], n->partial, nblocks, s);
+  GradOut out{{n->grad[0], n->grad[1], n->grad[2]}};
+  hipLaunchKernelGGL(k_wgrad_reduce, dim3((GSZ + 15) / 16, NLAYER), dim3(256), 0, s, n->partial,
+                     wgrad_groups(nblocks), stride, out);
+}
+
+void adam(Net* n, float lr, hipStream_t s) {
+  const float b1 = 0.9f, b2 = 0.999f, eps = 1e-8f;
+  n->step += 1;
+  const float bc1 = 1.f - std::pow(b1, (float)n->step);
+  const float bc2 = 1.f - std::pow(b2, (float)n->step);
+  AdamLayers a;
+  for (int l = 0; l < NLAYER; ++l)
+    a.l[l] = AdamLayer{n->p[l],  n->m[l],  n->v[l],    n->grad[l], n->wf[l],
+                       n->wb[l], n->bias[l], n->cin[l], n->cout[l]};
+  hipLaunchKernelGGL(k_adam, dim3((PSZ + 255) / 256, NLAYER), dim3(256), 0, s, a, lr, b1, b2, eps,
+                     bc1, bc2);
 }
 
 void sync_weights(Net* n, hipStream_t s) {
@@ -1281,7 +1395,8 @@ int sfac_conv3x3x3_wgrad_bf16_noalloc(const uint16_t* x, const uint16_t* gz, flo
 }
 
 size_t sfac_conv3x3x3_wgrad_partial_size(int nblocks) {
-  return nblocks <= 0 ? 0 : (size_t)wgrad_waves(nblocks * NROW) * GSZ;
+  // no less than any smaller block count needs
+  return nblocks <= 0 ? 0 : (size_t)std::min(4l * nblocks, (long)kWgradGroups) * GSZ;
 }
 
 int sfac_block_sor(const double* r, const double* dxf, const double* dyf, const double* dzf,
@@ -1332,7 +1447,9 @@ int sfac_learned_create(int max_blocks, unsigned long long seed, void** out) {
       n->gbuf[1] = dalloc<uint16_t>(ncells * CH);
       n->pred = dalloc<float>(ncells);
       n->scale = dalloc<double>(max_blocks);
-      n->partial = dalloc<float>((size_t)wgrad_waves(max_blocks * NROW) * GSZ);
+      // (a smaller batch may take more work-groups than the largest one)
+      n->partial = dalloc<float>((size_t)std::min(4l * max_blocks, (long)kWgradGroups) * NLAYER *
+                                 GSZ);
       n->loss_partial = dalloc<float>((ncells + 255) / 256);
       n->loss = dalloc<float>(1);
       n->unsaved = dalloc<int>(1);
@@ -1367,7 +1484,7 @@ int sfac_learned_features(void* net, const double* r, const double* logd, double
     need(r != nullptr, "null residual");
     need(h > 0.0, "h must be positive");
     if (nblocks == 0) return;
-    hipLaunchKernelGGL(k_features, dim3(nblocks), dim3(256), 0, stream, r, logd, 0.0, h * h,
+    hipLaunchKernelGGL(k_features, dim3(nblocks), dim3(kFeatThreads), 0, stream, r, logd, 0.0, h * h,
                        n->act[0], n->scale);
   });
 }
@@ -1416,14 +1533,7 @@ int sfac_learned_adam(void* net, float lr, hipStream_t stream) {
   return guarded([&] {
     Net* n = net_of(net, 0);
     save_hidden(n, stream);
-    const float b1 = 0.9f, b2 = 0.999f, eps = 1e-8f;
-    n->step += 1;
-    const float bc1 = 1.f - std::pow(b1, (float)n->step);
-    const float bc2 = 1.f - std::pow(b2, (float)n->step);
-    for (int l = 0; l < NLAYER; ++l)
-      hipLaunchKernelGGL(k_adam, dim3((PSZ + 255) / 256), dim3(256), 0, stream, n->p[l], n->m[l],
-                         n->v[l], n->grad[l], n->cin[l], n->cout[l], lr, b1, b2, eps, bc1, bc2,
-                         n->wf[l], n->wb[l], n->bias[l]);
+    adam(n, lr, stream);
   });
 }
 
@@ -1433,18 +1543,11 @@ int sfac_learned_train_step(void* net, const double* r, const double* logd, cons
     Net* n = net_of(net, nblocks);
     need(r && target, "null residual or target");
     need(h > 0.0 && nblocks > 0, "bad h or block count");
-    hipLaunchKernelGGL(k_features, dim3(nblocks), dim3(256), 0, stream, r, logd, 0.0, h * h,
+    hipLaunchKernelGGL(k_features, dim3(nblocks), dim3(kFeatThreads), 0, stream, r, logd, 0.0, h * h,
                        n->act[0], n->scale);
     forward(n, nblocks, stream);
     backward(n, target, nblocks, stream);
-    const float b1 = 0.9f, b2 = 0.999f, eps = 1e-8f;
-    n->step += 1;
-    const float bc1 = 1.f - std::pow(b1, (float)n->step);
-    const float bc2 = 1.f - std::pow(b2, (float)n->step);
-    for (int l = 0; l < NLAYER; ++l)
-      hipLaunchKernelGGL(k_adam, dim3((PSZ + 255) / 256), dim3(256), 0, stream, n->p[l], n->m[l],
-                         n->v[l], n->grad[l], n->cin[l], n->cout[l], lr, b1, b2, eps, bc1, bc2,
-                         n->wf[l], n->wb[l], n->bias[l]);
+    adam(n, lr, stream);
   });
 }
 

@@ -199,6 +199,30 @@ def test_block_sor_from_a_start_matches_oracle(torch_gpu, blocks, sweeps, omega,
     assert np.abs(e - eo).max() <= 64 * 2.0 ** -52 * max(1, sweeps) * top
 
 
+@pytest.mark.parametrize("blocks", [1, 3, 127, 128, 600])
+def test_weight_gradient_matches_64_bit_sums(torch_gpu, blocks):
+    """Quarters of a block per work-group, whole blocks, and several blocks per
+    work-group, against float64 sums over shifted cells.  FP32 accumulation
+    over N = 4096 blocks terms in chains of at most N / 4 and sums of those:
+    the error is within N 2^-24 times the sum of the terms' sizes, and far
+    below in the 2-norm, where roundings average: 1e-5."""
+    torch = torch_gpu
+    from samrai_amd import learned as SL
+    _say("weight gradient, %d blocks" % blocks)
+    g = torch.Generator(device="cuda").manual_seed(blocks)
+    kw = dict(generator=g, device="cuda")
+    x, gz = (torch.randn((blocks, 16, 16, 16, 16), **kw).bfloat16() for _ in range(2))
+    got = SL.conv3x3x3_wgrad(torch, x.view(torch.int16), gz.view(torch.int16)).double()
+    pad = torch.nn.functional.pad(x.double(), (0, 0, 1, 1, 1, 1, 1, 1))
+    gt = gz.double().reshape(-1, 16).t().contiguous()
+    for t in range(27):
+        z, y, q = t // 9, (t // 3) % 3, t % 3
+        ref = gt @ pad[:, z:z + 16, y:y + 16, q:q + 16].reshape(-1, 16)
+        assert torch.linalg.norm(got[t] - ref) <= 1e-5 * torch.linalg.norm(ref), t
+    bias = gt.sum(1)
+    assert torch.linalg.norm(got[27][:, 0] - bias) <= 1e-5 * torch.linalg.norm(bias)
+
+
 @pytest.mark.parametrize("blocks", [1, 63, 256, 300])
 def test_backward_after_a_correction_equals_backward_after_forward(torch_gpu, blocks):
     """A correction does not store the hidden activations, a forward pass
