@@ -637,7 +637,7 @@ int CellPoissonFACOps::smoothFused(PatchDataSet& e, const PatchDataSet& r, int l
   PatchDataSet& tmp = *d_fused_tmp;
   const double* Ds = d_spec.dIsConstant() ? nullptr : d_spec.getD()->slab(ln);
   const double* Cs = d_spec.cMode() == 2 ? d_spec.getC()->slab(ln) : nullptr;
-  ghostFill(e, ln, true, true, false);
+  if (!d_fills.zero_start) ghostFill(e, ln, true, true, false);
   const double launch_bytes = (d_spec.dIsConstant() ? 24.0 : 48.0) * (double)T.ncells;
   for (int s = 0; s < num_sweeps; ++s) {
     const PatchDataSet& src = (s & 1) ? tmp : e;
@@ -663,7 +663,7 @@ int CellPoissonFACOps::smoothFused(PatchDataSet& e, const PatchDataSet& r, int l
   }
   if (num_sweeps & 1)
     sfac::launch_copy_interior(T.cells.launch(), T.geom, e.table(ln), tmp.table(ln), 1, d_stream);
-  ghostFill(e, ln, false, true, false);
+  if (!d_fills.skip_closing) ghostFill(e, ln, false, true, d_fills.lean);
   return num_sweeps;
 }
 
@@ -1131,7 +1131,7 @@ int CellPoissonFACOps::smoothBox(PatchDataSet& e, const PatchDataSet& r, int num
                          (check && num_sweeps > 0) ? d_stop + 1 : nullptr, num_sweeps, G, 0,
                          d_stream, B.fp32, e.elemBytes());
   // edges/corners too, as the reference's last NoCoarse fill does
-  ghostFill(e, ln, false, true, false);
+  if (!d_fills.skip_closing) ghostFill(e, ln, false, true, d_fills.lean);
   if (check && (maxres_out || d_logging)) {
     int sweeps = 0;
     double mr = 0.0;
@@ -1207,8 +1207,7 @@ int CellPoissonFACOps::smoothErrorByRedBlack(PatchDataSet& e, const PatchDataSet
   // (CellPoissonFACOps.C:1364-1373); above the coarsest level the fill with
   // the coarser level rewrites every ghost the fill without it sets, with
   // the same values, so it alone is run
-  if (ln > d_ln_min) ghostFill(e, ln, true, true, false);
-  else ghostFill(e, ln, false, true, false);
+  if (!d_fills.zero_start) ghostFill(e, ln, ln > d_ln_min, true, d_fills.lean);
   const int nsc = T.smooth.nchunks;
   double* red = tol >= 0.0 ? d_maxres[ln] : nullptr;
   double* blk = tol >= 0.0 ? d_maxres[ln] + nsc : nullptr;
@@ -1272,7 +1271,7 @@ int CellPoissonFACOps::smoothErrorByRedBlack(PatchDataSet& e, const PatchDataSet
                                (tol >= 0.0 && np > 0) ? &chk : nullptr, nullptr, 1);
   }
   // edges/corners too, as the reference's last NoCoarse fill does
-  ghostFill(e, ln, false, true, false);
+  if (!d_fills.skip_closing) ghostFill(e, ln, false, true, d_fills.lean);
   if (tol >= 0.0 && (maxres_out || d_logging)) {
     int sweeps = 0;
     double mr = 0.0;
@@ -1359,8 +1358,7 @@ int CellPoissonFACOps::smoothColourLP(PatchDataSet& e, const PatchDataSet& r, in
   const int elem = e.elemBytes();
   void* const* et = reinterpret_cast<void* const*>(e.table(ln));
   const sfac::RobinDev bc = robinDev();
-  if (ln > d_ln_min) ghostFill(e, ln, true, true, false);
-  else ghostFill(e, ln, false, true, false);
+  if (!d_fills.zero_start) ghostFill(e, ln, ln > d_ln_min, true, d_fills.lean);
   const int nsc = T.smooth.nchunks;
   double* red = tol >= 0.0 ? d_maxres[ln] : nullptr;
   double* blk = tol >= 0.0 ? d_maxres[ln] + nsc : nullptr;
@@ -1413,7 +1411,7 @@ int CellPoissonFACOps::smoothColourLP(PatchDataSet& e, const PatchDataSet& r, in
                                   nullptr, 1, bc, stop, d_stream,
                                   (tol >= 0.0 && np > 0) ? &chk : nullptr);
   }
-  ghostFill(e, ln, false, true, false);
+  if (!d_fills.skip_closing) ghostFill(e, ln, false, true, d_fills.lean);
   if (tol >= 0.0 && (maxres_out || d_logging)) {
     int sweeps = 0;
     double mr = 0.0;
@@ -1576,9 +1574,14 @@ int CellPoissonFACOps::solveCoarsestLevel(SAMRAIVectorReal& e, const SAMRAIVecto
       fail("CellPoissonFACOps: multigrid coarse solve on a level other than the coarsest");
     solveBoxMG(*e.data, *r.data);
   } else {
+    // the fill below repeats the smoothing's closing one
+    CycleFills& f = d_fills;
+    const bool skip = f.skip_closing;
+    f.skip_closing = f.lean;
     smoothErrorByRedBlack(*e.data, *r.data, coarsest_ln, d_coarse_max, d_coarse_tol);
+    f.skip_closing = skip;
   }
-  ghostFill(*e.data, coarsest_ln, false, true, false);
+  ghostFill(*e.data, coarsest_ln, false, true, d_fills.lean);
   return 0;
 }
 
@@ -1592,7 +1595,8 @@ void CellPoissonFACOps::computeCompositeResidualOnLevel(SAMRAIVectorReal& r,
   // S1 ghost fill, S3 coarsened fine flux onto the faces it replaces, then
   // S2 (fluxes, formed on the fly) and S4 (residual, saved boundary flux)
   // in one pass
-  ghostFill(*u.data, ln, ln > d_ln_min, error_equation_indicator, false);
+  if (!d_fills.residual_filled)
+    ghostFill(*u.data, ln, ln > d_ln_min, error_equation_indicator, d_fills.lean);
   sfac::LevelGeom G = T.geom;
   if (ln < d_ln_max) {
     const auto& Tf = d_h.tables(ln + 1);
@@ -1618,7 +1622,7 @@ void CellPoissonFACOps::restrictSolution(const SAMRAIVectorReal& s, SAMRAIVector
   const auto& Tc = d_h.tables(dest_ln);
   sfac::launch_restrict(Tf.restrict_to_coarser.launch(), Tc.geom, Tf.geom, d.data->table(dest_ln),
                         d.data->ghost(), s.data->table(dest_ln + 1), s.data->ghost(), d_stream);
-  ghostFill(*d.data, dest_ln, dest_ln > d_ln_min, false, false);
+  if (!d_fills.lean) ghostFill(*d.data, dest_ln, dest_ln > d_ln_min, false, false);
 }
 
 void CellPoissonFACOps::restrictResidual(const SAMRAIVectorReal& s, SAMRAIVectorReal& d,

@@ -183,6 +183,22 @@ class CellPoissonFACOps : public FACOperatorStrategy {
   // solveCoarsestLevel end with that fill, so FACPreconditioner's recursive
   // cycle, which prolongs right after them, sets this around the call.
   void setProlongCoarseFilled(bool on) { d_prolong_coarse_filled = on; }
+  // Which ghost fills the operations of a solve's own cycle leave out.  A
+  // single operation (the defaults) fills every ghost it may need and leaves
+  // all of them filled, as the reference's schedules do; inside a cycle whose
+  // operators read face ghosts only (leanFillsUsable) edges and corners are
+  // never read, and most face fills repeat the one before them.
+  struct CycleFills {
+    bool lean = false;           // faces only; restricted solutions are not refilled
+    bool zero_start = false;     // smoothing: e is 0 with its ghosts on both levels
+    bool skip_closing = false;   // smoothing: nothing reads the ghosts afterwards
+    bool residual_filled = false;  // residual: smoothing just ended with its fill
+  };
+  CycleFills& cycleFills() { return d_fills; }
+  bool leanFillsUsable() const {
+    return d_cf_method == sfac::kProlongConstant && d_prolongation != "LINEAR_REFINE" &&
+           !learnedActive();
+  }
   // 16^3 windows covering level ln's patches (device, 8 ints each) for the
   // learned correction; count = the number of windows.
   const int* learnedWindows(int ln, int* count);
@@ -346,6 +362,7 @@ class CellPoissonFACOps : public FACOperatorStrategy {
   void mgBottom(int columns, double* e);
   bool d_mg_small_direct = false;
   bool d_prolong_coarse_filled = false;
+  CycleFills d_fills;
   std::vector<int*> d_lwin;  // learned-correction windows per level (device)
   std::vector<int> d_lwin_n;
   double* d_mg_partial = nullptr;
@@ -469,6 +486,7 @@ class FACPreconditioner {
   void runCycle(SAMRAIVectorReal& u);
   void allocateTmpError();
   // one cycle of solveSystem up to the residual norm's device reductions
+  bool leanCycle() const;
   void enqueueCycle(SAMRAIVectorReal& u, SAMRAIVectorReal& f);
   void releaseCycleGraph();
   // captured cycles, [0] without and [1] with the learned correction
