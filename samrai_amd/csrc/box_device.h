@@ -167,6 +167,14 @@ __device__ inline T cell_update(T* U, int q, int SY, int SZd, int SZu, const Coe
   return fabs(residual);
 }
 
+// Raise the word at p (the bits of a non-negative double) to m.  Hundreds of
+// work-groups raise one word and most of them to less than it holds: those
+// only read it.
+__device__ inline void raise_max(unsigned long long* p, double m) {
+  const unsigned long long bits = (unsigned long long)__double_as_longlong(m);
+  if (__hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) < bits) atomicMax(p, bits);
+}
+
 // DIM, DVAR and CMODE of a level's arrays as template arguments of F::run.
 template <template <int, bool, int> class F, typename T, class... Args>
 void dispatch3(const BoxLevel& G, const BoxArraysT<T>& A, Args&&... args) {

@@ -122,6 +122,38 @@ void launch_box_lds_rbgs(const BoxLevel& G, const BoxArrays& A, const RobinDev& 
                          const double* uin, double* e0, double* e1, int sweeps,
                          const BoxCheck& K, int check, hipStream_t s);
 
+// ---- two sweeps per launch on levels too large for that (box_pair.hip) ----
+// Early-exit data of launch number `launch` of a smoothing call.  slots: six
+// words (nullptr without a tolerance), two per launch of three; a launch
+// raises its two to the max |residual| of its sweeps over the last patch,
+// reads those of the launch before it (which took `prev` sweeps) and clears
+// those of the next.  When that launch met the tolerance it records stop,
+// sweeps, maxres_out and buffer (0: the result is in the buffer launch 0 read,
+// 1: in the other), after repeating a first sweep that already met it; final:
+// the launch after the last sweeps, which records in any case and sweeps no
+// further.
+struct PairCheck {
+  unsigned long long* slots;
+  int launch, prev, final;
+  double tol;
+  int* stop;
+  int* sweeps;
+  int* buffer;
+  double* maxres_out;
+};
+// Levels (cells) on which a launch of two sweeps is faster than two launches,
+// us per sweep with variable D: 3-D 48^3 5.7 (singly 6.3), 64^3 10.4 (7.4);
+// 2-D up to the largest measured, 500^2 3.5 (6.0).  On small 3-D levels 8x8x4
+// tiles give the machine more work-groups than 8x8x8 ones: 32^3 has 128 with
+// the one, 64 with the other; from 45 x 58 x 39 on there are enough of both and
+// 8x8x4 only adds redundant cells (9.8 against 5.7).
+constexpr long kPairCells3 = 150000, kPairCells2 = 300000, kPairSmallTile = 40000;
+bool box_pair_pays(const BoxLevel& G);
+// One or two sweeps from A.ein (nullptr: 0) to A.eout; without slots nothing
+// is done once *K.stop is set.
+void launch_box_pair(const BoxLevel& G, const BoxArrays& A, const RobinDev& bc,
+                     const PairCheck& K, int sweeps, hipStream_t s);
+
 // The lower part of a multigrid V-cycle in one launch, over the n levels G
 // (each half the one before) with arrays A (r of the first is its right-hand
 // side): pre-sweeps, residual restriction, ..., `last` sweeps from 0 on the

@@ -254,7 +254,7 @@ k_box_rbgs(BoxLevel G, BoxArraysT<T> A, RobinDev bc, int homogeneous, BoxCheck K
     if (meets) {  // uniform over the work-group
       mr = block_max(mr, wm);
       if (threadIdx.x == 0)
-        atomicMax(K.slots + K.sweep % 3, (unsigned long long)__double_as_longlong(mr));
+        raise_max(K.slots + K.sweep % 3, mr);
     }
   }
 }

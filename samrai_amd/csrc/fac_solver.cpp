@@ -202,7 +202,7 @@ using pdat::PatchDataSet;
 
 CellPoissonFACOps::CellPoissonFACOps(hier::PatchHierarchy& h, hipStream_t stream)
     : d_h(h), d_stream(stream) {
-  hip_check(hipMalloc(&d_stop, sizeof(int) * 2), "hipMalloc(stop)");
+  hip_check(hipMalloc(&d_stop, sizeof(int) * 3), "hipMalloc(stop)");
   hip_check(hipMalloc(&d_scalars, sizeof(double) * 4), "hipMalloc(scalars)");
   hip_check(hipHostMalloc(&h_pinned, sizeof(double) * 4), "hipHostMalloc");
 }
@@ -742,8 +742,8 @@ void CellPoissonFACOps::setupBoxPath() {
   hip_check(hipMalloc(&B.e[0], sizeof(double) * vol), "hipMalloc(box e)");
   hip_check(hipMalloc(&B.e[1], sizeof(double) * vol), "hipMalloc(box e)");
   hip_check(hipMalloc(&B.r, sizeof(double) * vol), "hipMalloc(box r)");
-  // early-exit maxima of three consecutive sweeps (BoxCheck)
-  hip_check(hipMalloc(&B.slots, sizeof(double) * 4), "hipMalloc(box slots)");
+  // early-exit maxima of three consecutive sweeps (BoxCheck) or pairs (PairCheck)
+  hip_check(hipMalloc(&B.slots, sizeof(double) * 6), "hipMalloc(box slots)");
   hip_check(hipMalloc(&B.mismatch, sizeof(int)), "hipMalloc(box flag)");
   if (d_spec.cMode() == 2) hip_check(hipMalloc(&B.C, sizeof(double) * vol), "hipMalloc(box C)");
   B.ok = true;
@@ -927,6 +927,10 @@ void CellPoissonFACOps::mgSweeps(int m, int n, bool zero_in) {
                               d_stream);
     return;
   }
+  if (n > 0 && n % 4 == 0 && mgPair(m)) {  // whole pairs of launches end in e[0]
+    for (int s = 0; s < n / 2; ++s) mgPairSweeps(m, s & 1, s == 0 && zero_in);
+    return;
+  }
   if (zero_in && n == 0) {
     const int dim = d_h.dim();
     const long nc = (long)L.G.n[0] * L.G.n[1] * (dim == 3 ? L.G.n[2] : 1);
@@ -937,6 +941,23 @@ void CellPoissonFACOps::mgSweeps(int m, int n, bool zero_in) {
     A.eout = L.e[(s + 1) & 1];
     sfac::launch_box_rbgs(L.G, A, bc, 1, K, mgVariant(m), d_stream);
   }
+}
+
+// Does multigrid level m take two sweeps per launch?  Then one such launch
+// from buffer `from` (zero: from 0) to the other.
+bool CellPoissonFACOps::mgPair(int m) const {
+  return d_box_variant < 0 && sfac::box_pair_pays(d_mg[m].G) &&
+         !sfac::box_lds_fits(d_mg[m].G, mgArrays(m));
+}
+
+void CellPoissonFACOps::mgPairSweeps(int m, int from, bool zero) {
+  MGLevel& L = d_mg[m];
+  sfac::BoxArrays A = mgArrays(m);
+  A.ein = zero ? nullptr : L.e[from];
+  A.eout = L.e[1 - from];
+  sfac::PairCheck P{};
+  P.stop = d_mg_flag;
+  sfac::launch_box_pair(L.G, A, robinDev(), P, 2, d_stream);
 }
 
 // Tile shape of multigrid level m's sweeps: the tuned one on the finest level
@@ -983,12 +1004,19 @@ void CellPoissonFACOps::mgVcycle(int m) {
     mgSweeps(m, kMGLastSweeps, m > 0);
     return;
   }
-  mgSweeps(m, kMGPre, m > 0);
+  // two sweeps per launch: the pre-smoothing ends in e[1], the post-smoothing
+  // takes that back to e[0]
+  static_assert(kMGPre == 2 && kMGPost == 2, "one launch of two sweeps each");
+  const bool pair = mgPair(m);
+  if (pair) mgPairSweeps(m, 0, m > 0);
+  else mgSweeps(m, kMGPre, m > 0);
+  double* e = L.e[pair ? 1 : 0];
   MGLevel& C = d_mg[m + 1];
-  sfac::launch_mg_restrict_residual(L.G, mgArrays(m), bc, L.e[0], C.G, C.f, d_mg_flag, d_stream);
+  sfac::launch_mg_restrict_residual(L.G, mgArrays(m), bc, e, C.G, C.f, d_mg_flag, d_stream);
   mgVcycle(m + 1);
-  sfac::launch_mg_prolong_add(C.G, bc, C.e[0], L.G, L.e[0], d_mg_flag, d_stream, d_box.fp32);
-  mgSweeps(m, kMGPost);
+  sfac::launch_mg_prolong_add(C.G, bc, C.e[0], L.G, e, d_mg_flag, d_stream, d_box.fp32);
+  if (pair) mgPairSweeps(m, 1, false);
+  else mgSweeps(m, kMGPost);
 }
 
 void CellPoissonFACOps::solveBoxMG(PatchDataSet& e, const PatchDataSet& r) {
@@ -1107,7 +1135,33 @@ int CellPoissonFACOps::smoothBox(PatchDataSet& e, const PatchDataSet& r, int num
   const bool lds = num_sweeps > 0 && d_box_variant < 0 && sfac::box_lds_fits(G, A);
   if (lds)
     sfac::launch_box_lds_rbgs(G, A, bc, B.e[0], B.e[0], B.e[1], num_sweeps, K, check, d_stream);
-  for (int s = 0; s < num_sweeps && !lds; ++s) {
+  // a larger one on which a launch is mostly latency takes two sweeps per
+  // launch; the buffer of the result is then counted in launches
+  const bool pair =
+      num_sweeps > 0 && d_box_variant < 0 && !lds && sfac::box_pair_pays(G);
+  const int npair = (num_sweeps + 1) / 2;
+  if (pair) {
+    sfac::PairCheck P{};
+    P.tol = tol;
+    P.maxres_out = d_scalars + 1;
+    if (check) {
+      sfac::launch_fill_int(d_stop + 2, 1, 0, d_stream);
+      sfac::launch_fill(B.slots, 6, 0.0, d_stream);
+      P.slots = reinterpret_cast<unsigned long long*>(B.slots);
+      P.stop = d_stop;
+      P.sweeps = d_stop + 1;
+      P.buffer = d_stop + 2;
+    }
+    for (int l = 0; l < npair + (check ? 1 : 0); ++l) {
+      P.launch = l;
+      P.final = l == npair;
+      P.prev = l == npair && (num_sweeps & 1) ? 1 : 2;
+      A.ein = B.e[l & 1];
+      A.eout = B.e[(l + 1) & 1];
+      sfac::launch_box_pair(G, A, bc, P, l + 1 == npair && (num_sweeps & 1) ? 1 : 2, d_stream);
+    }
+  }
+  for (int s = 0; s < num_sweeps && !lds && !pair; ++s) {
     K.sweep = s;
     A.ein = B.e[s & 1];
     A.eout = B.e[(s + 1) & 1];
@@ -1122,14 +1176,14 @@ int CellPoissonFACOps::smoothBox(PatchDataSet& e, const PatchDataSet& r, int num
     tl.bytes = launch_bytes * num_sweeps;
     d_timed.push_back(tl);
   }
-  if (check && num_sweeps > 0 && !lds) {
+  if (check && num_sweeps > 0 && !lds && !pair) {
     sfac::launch_box_final_check(K, num_sweeps, d_stream);
   }
   // the sweeps done (known on the device when the loop may stop early)
   // select the buffer holding the result
   sfac::launch_box_cells(T.cells.launch(), T.geom, e.table(ln), e.ghost(), B.e[0], B.e[1],
-                         (check && num_sweeps > 0) ? d_stop + 1 : nullptr, num_sweeps, G, 0,
-                         d_stream, B.fp32, e.elemBytes());
+                         (check && num_sweeps > 0) ? d_stop + (pair ? 2 : 1) : nullptr,
+                         pair ? npair : num_sweeps, G, 0, d_stream, B.fp32, e.elemBytes());
   // edges/corners too, as the reference's last NoCoarse fill does
   if (!d_fills.skip_closing) ghostFill(e, ln, false, true, d_fills.lean);
   if (check && (maxres_out || d_logging)) {

@@ -359,6 +359,8 @@ class CellPoissonFACOps : public FACOperatorStrategy {
   bool d_mg_use_dense = false;
   int mgCells(int m) const;
   int mgVariant(int m) const;
+  bool mgPair(int m) const;
+  void mgPairSweeps(int m, int from, bool zero);
   void mgBottom(int columns, double* e);
   bool d_mg_small_direct = false;
   bool d_prolong_coarse_filled = false;

@@ -1,5 +1,6 @@
-"""Coarsest levels that one work-group holds in LDS: sweeps and early exit
-against the patch-wise passes and the grid-parallel sweep, bit for bit."""
+"""Coarsest levels that one work-group holds in LDS or that take two sweeps per
+launch: sweeps and early exit against the patch-wise passes and the
+grid-parallel sweep, bit for bit."""
 import numpy as np
 import pytest
 
@@ -68,7 +69,10 @@ def solve(case, data, spec, keys, fused, variant, bits):
 # odd rows, one-cell-wide and thin domains
 SIZES = [(3, 2, 2), (1, 5, 7), (9, 10, 11), (13, 17, 15), (16, 16, 16), (17, 16, 16), (32, 16, 16),
          (34, 16, 16), (2, 40, 40), (5, 3), (31, 23), (64, 64), (65, 64), (90, 91), (128, 64),
-         (130, 64), (300, 9)]
+         (130, 64), (300, 9),
+         # two sweeps per launch: both 3-D tiles, ragged ends of each, a last
+         # patch smaller than a tile's halo, and the first size past the rule
+         (33, 31, 35), (37, 41, 29), (6, 70, 40), (54, 53, 53), (251, 130)]
 
 
 @pytest.mark.parametrize("spec", [dict(dvar=False, cmode=0, robin=False),
@@ -83,7 +87,8 @@ def test_lds_sweeps_are_bit_identical(gpu_lib, n, spec):
     tolerance that stops the loop and one that does not."""
     case = one_level(*n)
     data = hc.make_data(case, seed=sum(n))
-    for sweeps, tol in ((7, 1e-300), (40, 0.5)):
+    # (13, 0.9) and (40, 0.5) stop after odd and even sweeps on different sizes
+    for sweeps, tol in ((7, 1e-300), (40, 0.5), (13, 0.9), (8, 1e-300)):
         print("lds sweeps", case["name"], spec, sweeps, tol, flush=True)
         keys = dict(coarse_solver_max_iterations=sweeps, coarse_solver_tolerance=tol)
         for bits, fused, variant in ((64, False, 0), (32, True, 0)):
