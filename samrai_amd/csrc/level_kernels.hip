@@ -222,7 +222,13 @@ k_ghost_items(const BoxItem* items, const Chunk* chunks, LevelGeom L, double* co
 // compflux*, :10-133, formed on the fly).  Work-group = one chunk of rows
 // (j,k) of one patch; the colour cells of a row lie on consecutive lanes, so
 // neighbour loads are fixed offsets from one 32-bit row base.  EWING: the
-// coarse-fine face fluxes come from the pre-pass snapshot L.cf_flux.
+// coarse-fine face fluxes come from the pre-pass snapshot L.cf_flux; flags and
+// fluxes of all of a cell's boundary faces are read at once and ahead of the
+// cell's own data, where one face after the other waited for its flag and then
+// its flux.  Memory bounds the pass: every line of u, f and D is read for each
+// colour (4.0 M cells, variable D: 192 MB in 37 us, 5 TB/s), so the reordering
+// gave little (two sweeps of that level 366 -> 360 us, the 54 M cell solve
+// 260 -> 257 ms).
 template <int DIM, bool DVAR, int CMODE, bool EWING>
 __global__ void __launch_bounds__(kThreads)
 k_rbgs(const BoxItem* items, const Chunk* chunks, LevelGeom L, double* const* e, int eg,
@@ -249,12 +255,20 @@ k_rbgs(const BoxItem* items, const Chunk* chunks, LevelGeom L, double* const* e,
   const int dys1 = nx + 2 * dgw, dys2 = dys1 * (ny + 1 + 2 * dgw);
   const int dzs1 = nx + 2 * dgw, dzs2 = dzs1 * (ny + 2 * dgw);
   const int cs1 = nx + 2 * ps.cghost, cs2 = cs1 * (ny + 2 * ps.cghost);
-  double* __restrict__ u = e[p];
-  const double* __restrict__ f = rhs[p];
-  const double* __restrict__ Dx = DVAR ? ps.D[0][p] : nullptr;
-  const double* __restrict__ Dy = DVAR ? ps.D[1][p] : nullptr;
-  const double* __restrict__ Dz = (DVAR && DIM == 3) ? ps.D[2][p] : nullptr;
-  const double* __restrict__ Cp = CMODE == 2 ? ps.C[p] : nullptr;
+  const auto u = gmem(e[p]);
+  const auto f = gmem(rhs[p]);
+  const auto Dx = gmem(DVAR ? ps.D[0][p] : nullptr);
+  const auto Dy = gmem(DVAR ? ps.D[1][p] : nullptr);
+  const auto Dz = gmem((DVAR && DIM == 3) ? ps.D[2][p] : nullptr);
+  const auto Cp = gmem(CMODE == 2 ? ps.C[p] : nullptr);
+  // per-face table offsets of the patch (-1: no coarse-fine part on it)
+  long cfo[6] = {-1, -1, -1, -1, -1, -1};
+  if (EWING) {
+#pragma unroll
+    for (int fc = 0; fc < 2 * DIM; ++fc) cfo[fc] = L.cf_off[p * 6 + fc];
+  }
+  const auto cff = gmem((const double*)L.cf_flux);
+  const auto cfg = gmem(L.cf);
   const double dxi = 1.0 / L.dx[0], dyi = 1.0 / L.dx[1];
   const double dzi = DIM == 3 ? 1.0 / L.dx[2] : 0.0;
   const double dxi2 = dxi * dxi, dyi2 = dyi * dyi, dzi2 = dzi * dzi;
@@ -268,8 +282,20 @@ k_rbgs(const BoxItem* items, const Chunk* chunks, LevelGeom L, double* const* e,
     const int par = DIM == 3 ? fmod2(b.lo[0] + j + k) : fmod2(b.lo[1] + j);
     const int ii = (par != colour ? 1 : 0) + 2 * m;
     if (ii >= nx) continue;
-    const int i = b.lo[0] + ii;
     const int o = (ii + eg) + us1 * (jj + eg) + us2 * (DIM == 3 ? kk + eg : 0);
+    // the snapshot flux of each patch-boundary face, with its flag
+    unsigned char cfb[6] = {0, 0, 0, 0, 0, 0};
+    double cfv[6] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
+    if (EWING) {
+      const int at[3] = {jj + ny * kk, ii + nx * kk, ii + nx * jj};
+      const bool on[6] = {ii == 0, ii == nx - 1, jj == 0, jj == ny - 1, kk == 0, kk == nz - 1};
+#pragma unroll
+      for (int fc = 0; fc < 2 * DIM; ++fc)
+        if (on[fc] && cfo[fc] >= 0) {
+          cfb[fc] = cfg[cfo[fc] + at[fc >> 1]];
+          cfv[fc] = cff[cfo[fc] + at[fc >> 1]];
+        }
+    }
     const double uc = u[o];
     // face fluxes: x at i and i+1, y at j and j+1, z at k and k+1
     double Dxl, Dxh, Dyl, Dyh, Dzl = 0.0, Dzh = 0.0;
@@ -298,14 +324,13 @@ k_rbgs(const BoxItem* items, const Chunk* chunks, LevelGeom L, double* const* e,
       fzh = dzi * Dzh * (u[o + us2] - uc);
     }
     if (EWING) {
-      int c[3] = {i, j, k};
-      if (ii == 0) { long x = cf_index(L, p, 0, c, b); if (x >= 0) fxl = L.cf_flux[x]; }
-      if (ii == nx - 1) { long x = cf_index(L, p, 1, c, b); if (x >= 0) fxh = L.cf_flux[x]; }
-      if (jj == 0) { long x = cf_index(L, p, 2, c, b); if (x >= 0) fyl = L.cf_flux[x]; }
-      if (jj == ny - 1) { long x = cf_index(L, p, 3, c, b); if (x >= 0) fyh = L.cf_flux[x]; }
+      if (cfb[0]) fxl = cfv[0];
+      if (cfb[1]) fxh = cfv[1];
+      if (cfb[2]) fyl = cfv[2];
+      if (cfb[3]) fyh = cfv[3];
       if (DIM == 3) {
-        if (kk == 0) { long x = cf_index(L, p, 4, c, b); if (x >= 0) fzl = L.cf_flux[x]; }
-        if (kk == nz - 1) { long x = cf_index(L, p, 5, c, b); if (x >= 0) fzh = L.cf_flux[x]; }
+        if (cfb[4]) fzl = cfv[4];
+        if (cfb[5]) fzh = cfv[5];
       }
     }
     double scal;
