@@ -82,7 +82,7 @@ __device__ inline T small_at(const T* E, const BoxLevel& G, const Slots& S, int 
   return v;
 }
 
-// mg_prolong_value (box_kernels.hip) from LDS.
+// k_mg_prolong_add (box_kernels.hip) of one cell, from LDS.
 template <int DIM, typename T>
 __device__ inline T small_prolong(const T* E, const BoxLevel& G, const Slots& S,
                                   const SmallRobin<T>& R, int i, int j, int k) {
