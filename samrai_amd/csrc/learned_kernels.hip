@@ -171,10 +171,10 @@ __global__ __launch_bounds__(256) void k_conv(const uint16_t* __restrict__ x,
 // step i forms plane i + 2 of the first layer, plane i of the second, the tap
 // products of plane i - 2 of the third and the prediction of plane i - 3, all
 // from planes of earlier steps, so that one barrier a step is enough (it
-// waits for LDS only, the stores drain behind it).  Nothing but the features
-// and the result is in memory.  What bounds it are the LDS reads and, of a
-// block, the latency of its 64 KB of input, which is loaded while the block
-// before it is worked on:
+// waits for LDS only, the stores drain behind it).  The hidden activations are
+// written once, for a backward pass, and not read back here.  What bounds it
+// are the LDS reads and, of a block, the latency of its 64 KB of input, which is
+// loaded while the block before it is worked on:
 //   layer 1: K holds 16 taps x 2 channels, so 2 products a row;
 //   layer 2: a fragment (row y', taps dx = -1 and 0 of one dz, or dx = 1 of two)
 //     serves the three output rows y' - 1 .. y' + 1, 5 fragments a row and 15
@@ -182,7 +182,8 @@ __global__ __launch_bounds__(256) void k_conv(const uint16_t* __restrict__ x,
 //   layer 3: N holds the 9 (dy, dx) taps, K two dz, 2 products a row; the
 //     prediction is then 9 adds per cell.
 // A correction of 4096 blocks (features, three layers, correction) 1.66 ms as
-// five kernels, 0.58 ms so: 0.49 PFLOP/s of real channels, 1.7 TB/s.
+// five kernels, 0.63 ms so: 0.43 PFLOP/s of real channels, 3.3 TB/s (0.58 ms
+// without the hidden activations' stores).
 constexpr int FWD_THREADS = 512;
 constexpr int FP = HB * HB;          // cells of a halo-padded plane
 constexpr int FWD_F = HB * FP;       // words: features, two BF16 a cell, all planes
@@ -199,13 +200,11 @@ struct Forward {
   double* scale;
   const uint16_t* w[NLAYER];
   const float* bias[NLAYER];
-  uint16_t* act[2];      // hidden activations (SAVE)
+  uint16_t* act[2];      // hidden activations
   float* pred;
   double* e;             // omega * scale * prediction (FROM_R)
   double omega;
   int nblocks;
-  int* unsaved;          // blocks whose hidden activations were not stored
-  int only_unsaved;      // do nothing unless *unsaved covers the block
 };
 
 // Barrier that orders LDS accesses only.
@@ -213,11 +212,11 @@ __device__ inline void lds_barrier() {
   asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
 }
 
-// SAVE: store the hidden activations (training).  FROM_R: one work-group per
-// block at a time forms its scale and features from the residual and writes
-// the correction; else a work-group takes 16 / slabs planes of a block.
+// FROM_R: one work-group per block at a time forms its scale and features from
+// the residual and writes the correction; else a work-group takes 16 / slabs
+// planes of a block.
 // Work-group b takes slabs b, b + gridDim.x, ... of all.
-template <bool SAVE, bool FROM_R>
+template <bool FROM_R>
 __global__ __launch_bounds__(FWD_THREADS) void k_forward(Forward P, int slabs) {
   __shared__ __align__(16) unsigned char lds[FWD_LDS];
   uint32_t* F = reinterpret_cast<uint32_t*>(lds);
@@ -226,7 +225,7 @@ __global__ __launch_bounds__(FWD_THREADS) void k_forward(Forward P, int slabs) {
   float* G = reinterpret_cast<float*>(H2 + 4 * FWD_H);
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int cx = lane & 15, g = lane >> 4, half = g & 1, tsel = g >> 1;
-  const int nwork = P.only_unsaved ? *P.unsaved * slabs : P.nblocks * slabs;
+  const int nwork = P.nblocks * slabs;
   if ((int)blockIdx.x >= nwork) return;
   constexpr int NV = FROM_R ? NCELL / FWD_THREADS : 1;
   double rv[NV], lv[NV];
@@ -280,7 +279,6 @@ __global__ __launch_bounds__(FWD_THREADS) void k_forward(Forward P, int slabs) {
     w3[m] = __builtin_bit_cast(bf16x8, v);
   }
   const float b1 = P.bias[0][cx], b2 = P.bias[1][cx], b3 = P.bias[2][0];
-  if (P.unsaved && !P.only_unsaved && threadIdx.x == 0) *P.unsaved = SAVE ? 0 : P.nblocks;
   const int nz = NB / slabs;
   const int y0 = 2 * wave;  // this wave's rows
   uint16_t* h1 = reinterpret_cast<uint16_t*>(H1);
@@ -423,17 +421,15 @@ __global__ __launch_bounds__(FWD_THREADS) void k_forward(Forward P, int slabs) {
         if (FROM_R) P.e[c] = P.omega * scale * (double)p;
       }
       // hidden planes to memory: the first layer's plane i + 1, the second's i - 1
-      if (SAVE) {
-        const int c = threadIdx.x >> 1, hf = threadIdx.x & 1;
-        const int at = (((c >> 4) + 1) * HB + (c & 15) + 1) * 2 + hf;
-        const int za = i + 1, zb = i - 1;
-        if (za >= z0 && za < zend)
-          reinterpret_cast<uint4*>(P.act[0])[((size_t)b * NCELL + za * 256 + c) * 2 + hf] =
-              H1[(za & 3) * FWD_H + at];
-        if (zb >= z0 && zb < zend)
-          reinterpret_cast<uint4*>(P.act[1])[((size_t)b * NCELL + zb * 256 + c) * 2 + hf] =
-              H2[(zb & 3) * FWD_H + at];
-      }
+      const int c = threadIdx.x >> 1, hf = threadIdx.x & 1;
+      const int at = (((c >> 4) + 1) * HB + (c & 15) + 1) * 2 + hf;
+      const int za = i + 1, zb = i - 1;
+      if (za >= z0 && za < zend)
+        reinterpret_cast<uint4*>(P.act[0])[((size_t)b * NCELL + za * 256 + c) * 2 + hf] =
+            H1[(za & 3) * FWD_H + at];
+      if (zb >= z0 && zb < zend)
+        reinterpret_cast<uint4*>(P.act[1])[((size_t)b * NCELL + zb * 256 + c) * 2 + hf] =
+            H2[(zb & 3) * FWD_H + at];
       lds_barrier();
     }
   }
@@ -1020,7 +1016,6 @@ struct Net {
   float* loss_partial = nullptr;
   float* loss = nullptr;
   double* blk[3] = {};         // level gathers: residual, log D, correction
-  int* unsaved = nullptr;      // blocks of the last pass whose act[1..2] were not stored
   int step = 0;
   int attached = 0;            // solvers using the network (learned_attach)
   int cin[NLAYER] = {2, CH, CH};
@@ -1146,7 +1141,6 @@ Forward forward_args(Net* n, int nblocks) {
   P.act[1] = n->act[2];
   P.pred = n->pred;
   P.nblocks = nblocks;
-  P.unsaved = n->unsaved;
   return P;
 }
 
@@ -1155,14 +1149,12 @@ Forward forward_args(Net* n, int nblocks) {
 // (which form five more planes of each layer than they need alone).
 void forward(Net* n, int nblocks, hipStream_t s) {
   const int slabs = nblocks >= 256 ? 1 : 4;
-  hipLaunchKernelGGL((k_forward<true, false>), dim3(std::min(nblocks * slabs, kForwardGroups)),
+  hipLaunchKernelGGL(k_forward<false>, dim3(std::min(nblocks * slabs, kForwardGroups)),
                      dim3(FWD_THREADS), 0, s, forward_args(n, nblocks), slabs);
 }
 
 // Scale, features, prediction and correction e of every block from r and
-// log D.  The hidden activations, which only a backward pass reads, are not
-// stored; *unsaved says so on the device, so that a replayed graph of this
-// call says so too.
+// log D, with the buffers features + forward leave.
 void correction(Net* n, const double* r, const double* logd, double logd_const, double h2,
                 double omega, double* e, int nblocks, hipStream_t s) {
   Forward P = forward_args(n, nblocks);
@@ -1172,20 +1164,8 @@ void correction(Net* n, const double* r, const double* logd, double logd_const, 
   P.h2 = h2;
   P.omega = omega;
   P.e = e;
-  hipLaunchKernelGGL((k_forward<false, true>), dim3(std::min(nblocks, kForwardGroups)),
+  hipLaunchKernelGGL(k_forward<true>, dim3(std::min(nblocks, kForwardGroups)),
                      dim3(FWD_THREADS), 0, s, P, 1);
-}
-
-__global__ void k_set_int(int* p, int v) { *p = v; }
-
-// The hidden activations a correction left out, before anything that reads
-// them or changes the weights they come from.
-void save_hidden(Net* n, hipStream_t s) {
-  Forward P = forward_args(n, n->max_blocks);
-  P.only_unsaved = 1;
-  hipLaunchKernelGGL((k_forward<true, false>), dim3(std::min(n->max_blocks, kForwardGroups)),
-                     dim3(FWD_THREADS), 0, s, P, 1);
-  hipLaunchKernelGGL(k_set_int, dim3(1), dim3(1), 0, s, n->unsaved, 0);
 }
 
 // Loss and gradients of every layer (after forward on the same features).
@@ -1276,7 +1256,6 @@ void free_net(Net* n) {
   (void)hipFree(n->partial);
   (void)hipFree(n->loss_partial);
   (void)hipFree(n->loss);
-  (void)hipFree(n->unsaved);
   for (int k = 0; k < 3; ++k) (void)hipFree(n->blk[k]);
   delete n;
 }
@@ -1452,8 +1431,6 @@ int sfac_learned_create(int max_blocks, unsigned long long seed, void** out) {
                                  GSZ);
       n->loss_partial = dalloc<float>((ncells + 255) / 256);
       n->loss = dalloc<float>(1);
-      n->unsaved = dalloc<int>(1);
-      ck(hipMemset(n->unsaved, 0, sizeof(int)));
       for (int k = 0; k < 3; ++k) n->blk[k] = dalloc<double>(ncells);
       init_params(n, seed, 0);
       ck(hipStreamSynchronize(0));
@@ -1524,7 +1501,6 @@ int sfac_learned_backward(void* net, const double* target, int nblocks, hipStrea
     Net* n = net_of(net, nblocks);
     need(target != nullptr, "null target");
     need(nblocks > 0, "backward needs at least one block");
-    save_hidden(n, stream);
     backward(n, target, nblocks, stream);
   });
 }
@@ -1532,7 +1508,6 @@ int sfac_learned_backward(void* net, const double* target, int nblocks, hipStrea
 int sfac_learned_adam(void* net, float lr, hipStream_t stream) {
   return guarded([&] {
     Net* n = net_of(net, 0);
-    save_hidden(n, stream);
     adam(n, lr, stream);
   });
 }
@@ -1570,7 +1545,6 @@ int sfac_learned_set_params(void* net, const float* host) {
   return guarded([&] {
     Net* n = net_of(net, 0);
     need(host != nullptr, "null host buffer");
-    save_hidden(n, 0);
     for (int l = 0; l < NLAYER; ++l) {
       ck(hipMemcpy(n->p[l], host + (size_t)l * PSZ, PSZ * sizeof(float), hipMemcpyHostToDevice));
       ck(hipMemset(n->m[l], 0, PSZ * sizeof(float)));
