@@ -483,13 +483,18 @@ __global__ __launch_bounds__(256) void k_wgrad(const uint16_t* __restrict__ x,
   struct Cell {
     uint4 lo, hi;
   };
+  // the caller's arrays are aligned to their elements only; global memory takes
+  // a 16-byte load at any address, so this is one instruction either way
+  struct __attribute__((packed, aligned(2))) Channels {
+    uint32_t w[8];
+  };
   auto load = [&](const uint16_t* p, int b, int z) {  // plane z's cell of this thread
     Cell c{make_uint4(0u, 0u, 0u, 0u), make_uint4(0u, 0u, 0u, 0u)};
     if ((unsigned)z < (unsigned)NB) {
-      const uint4* q =
-          reinterpret_cast<const uint4*>(p + ((size_t)b * NCELL + z * 256 + threadIdx.x) * CH);
-      c.lo = q[0];
-      c.hi = q[1];
+      const Channels q = *reinterpret_cast<const Channels*>(
+          p + ((size_t)b * NCELL + z * 256 + threadIdx.x) * CH);
+      c.lo = make_uint4(q.w[0], q.w[1], q.w[2], q.w[3]);
+      c.hi = make_uint4(q.w[4], q.w[5], q.w[6], q.w[7]);
     }
     return c;
   };

@@ -223,6 +223,30 @@ def test_weight_gradient_matches_64_bit_sums(torch_gpu, blocks):
     assert torch.linalg.norm(got[27][:, 0] - bias) <= 1e-5 * torch.linalg.norm(bias)
 
 
+@pytest.mark.parametrize("shift", [1, 3, 4])
+def test_weight_gradient_takes_arrays_aligned_to_their_elements(torch_gpu, shift):
+    """Operands that start 2, 6 and 8 bytes past a 16-byte boundary give the
+    bits that the same operands on one give."""
+    torch = torch_gpu
+    from samrai_amd import learned as SL
+    _say("weight gradient, operands shifted by %d elements" % shift)
+    g = torch.Generator(device="cuda").manual_seed(shift)
+    n = 2 * 4096 * 16
+    bufs = [torch.randn(n + 8, generator=g, device="cuda").bfloat16().view(torch.int16)
+            for _ in range(2)]
+    grads = []
+    for k in (0, shift):
+        ops = []
+        for b in bufs:
+            full = torch.zeros(n + 8, dtype=torch.int16, device="cuda")
+            full[k:k + n] = b[:n]
+            ops.append(full[k:k + n].view(2, 16, 16, 16, 16))
+            assert ops[-1].data_ptr() % 16 == 2 * k
+        grads.append(SL.conv3x3x3_wgrad(torch, *ops))
+    assert grads[0].abs().max() > 0
+    assert torch.equal(*grads)
+
+
 @pytest.mark.parametrize("blocks", [1, 63, 256, 300])
 def test_state_after_a_correction_is_that_after_forward(torch_gpu, blocks):
     """A correction leaves the buffers that features, forward and correction
