@@ -8,6 +8,7 @@
 #include <chrono>
 #include <cmath>
 #include <cstdio>
+#include <typeinfo>
 
 #include "fac_solver.hpp"
 
@@ -265,9 +266,12 @@ void FACPreconditioner::enqueueCycle(SAMRAIVectorReal& u, SAMRAIVectorReal& f) {
 // The recursive cycle leaves out the ghost fills nothing reads or that repeat
 // one before them (54 M cells, four levels: 296 -> 260 ms a solve; a
 // 0.2 M cell two-level solve 3.58 -> 2.34 ms); a solve then ends with a
-// full fill of u.
+// full fill of u and e.  Operators derived from the library's may read the
+// ghosts that theirs do not, in an operation or after a cycle: they get the
+// full sequence.
 bool FACPreconditioner::leanCycle() const {
-  return d_algorithm == "default" && d_gpu->leanFillsUsable();
+  return d_algorithm == "default" && typeid(d_ops) == typeid(CellPoissonFACOps) &&
+         d_gpu->leanFillsUsable();
 }
 
 void FACPreconditioner::runOneCycle(SAMRAIVectorReal& u) {
@@ -360,10 +364,13 @@ bool FACPreconditioner::solveSystem(SAMRAIVectorReal& u, SAMRAIVectorReal& f) {
     d_avg_factor = std::pow(d_net_factor, 1.0 / d_iterations);
     d_ops.postprocessOneCycle(d_iterations - 1, u, d_r);
   } while (d_residual_norm > eff && d_iterations < d_max_cycles);
-  // u's edge and corner ghosts, which a lean cycle does not set
+  // the ghosts that a lean cycle does not set: edges and corners, and those of
+  // the finest level's last smoothing
   if (leanCycle())
-    for (int ln = d_lmax; ln >= d_lmin; --ln)
+    for (int ln = d_lmax; ln >= d_lmin; --ln) {
       d_gpu->ghostFill(*u.data, ln, ln > d_lmin, false, false);
+      d_gpu->ghostFill(*d_e.data, ln, ln > d_lmin, true, false);
+    }
   hip_check(hipStreamSynchronize(d_gpu->stream()), "hipStreamSynchronize");
   d_seconds = std::chrono::duration<double>(std::chrono::steady_clock::now() - t0).count();
   if (clear_when_done) deallocateSolverState();
