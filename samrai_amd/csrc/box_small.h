@@ -23,8 +23,8 @@
 // value, the one a ghost fill of the current state writes there.
 //
 // Measured, us per sweep with the early-exit test, FP64, in place of one launch
-// of k_box_rbgs: 64 x 64 constant D 1.51 (4.42), 31 x 23 1.18 (4.54), 16^3
-// variable D 3.36 (8.99), 8^3 0.82 (9.15).
+// of k_box_rbgs: 64 x 64 constant D 1.52 (4.69), 31 x 23 1.00 (4.70), 16^3
+// variable D 3.05 (9.35), 9^3 1.28 (8.65).
 #pragma once
 
 #include <cmath>
@@ -41,11 +41,13 @@ namespace {
 // 512 threads and four cells each).
 constexpr int kSmallThreads(bool coefs) { return coefs ? 512 : 1024; }
 
-// The homogeneous Robin ghost of every boundary side as c1 u / c2 (robin_ghost):
-// the coefficients and the reciprocal of c2; per location a bit of `exact`
-// when both are powers of two (Dirichlet and Neumann data on grids of such
-// spacing), so that u times their ratio (in rc) has the same bits, and of
-// `quick` when the quotient may be formed with the reciprocal.
+// The homogeneous Robin ghost of every boundary side as c1 u / c2 (robin_ghost).
+// exact: every side's coefficients are powers of two (Dirichlet and Neumann
+// data on grids of such spacing), so that u times their ratio, then in rc, has
+// the same bits; else rc is the reciprocal of c2, and with `quick` every
+// side's quotient may be formed with it.  One choice for all sides: made side
+// by side inside the ghosts it cost more than the quotient saves (64 sweeps of
+// 5^3 83 us, 55 us so, 67 us with plain divisions).
 template <typename T>
 struct SmallRobin {
   T c1[6], c2[6], rc[6];
@@ -56,20 +58,20 @@ template <typename T>
 SmallRobin<T> small_robin(const BoxLevel& G, const RobinDev& bc) {
   SmallRobin<T> R{};
   const T half = (T)0.5;
+  R.exact = R.quick = 1;
   for (int loc = 0; loc < 2 * G.dim; ++loc) {
     const T h = (T)G.dx[loc >> 1], av = (T)bc.a[loc], bv = (T)bc.b[loc];
     R.c1[loc] = bv - half * h * av;
     R.c2[loc] = bv + half * h * av;
-    const double m = R.c2[loc] < 0 ? -(double)R.c2[loc] : (double)R.c2[loc];
-    R.rc[loc] = m > 0 ? (T)1 / R.c2[loc] : (T)0;
-    if (m > 1e-8 && m < 1e8) R.quick |= 1 << loc;
+    const double m = std::fabs((double)R.c2[loc]);
     int ex;
-    if ((R.quick >> loc & 1) && std::fabs(std::frexp((double)R.c1[loc], &ex)) == 0.5 &&
-        std::frexp(m, &ex) == 0.5) {
-      R.exact |= 1 << loc;
-      R.rc[loc] = R.c1[loc] / R.c2[loc];
-    }
+    if (!(m > 1e-8 && m < 1e8)) R.quick = 0;
+    if (std::fabs(std::frexp((double)R.c1[loc], &ex)) != 0.5 || std::frexp(m, &ex) != 0.5)
+      R.exact = 0;
   }
+  if (!R.quick) R.exact = 0;
+  for (int loc = 0; loc < 2 * G.dim; ++loc)
+    R.rc[loc] = R.exact ? R.c1[loc] / R.c2[loc] : (R.quick ? (T)1 / R.c2[loc] : (T)0);
   return R;
 }
 
@@ -89,21 +91,24 @@ __device__ inline float fused(float a, float b, float c) { return fmaf(a, b, c);
 // c1 u / c2 for a u in quick_range: correctly rounded from rc = 1 / c2
 // correctly rounded by a quotient estimate and two residual corrections with
 // fused multiply-adds, the second of which rounds correctly (Markstein, IBM
-// J. Res. Dev. 34, 1990); with `exact`, u times the ratio in rc.
+// J. Res. Dev. 34, 1990).
 template <int DIM, typename T>
 __device__ inline T quick_ghost(const SmallRobin<T>& R, int loc, T u) {
-  if ((R.exact >> loc) & 1) return u * R.rc[loc];
-  const T c = R.c2[loc], rc = R.rc[loc];
   const T p = DIM == 3 ? (T)0 + u * R.c1[loc] : u * R.c1[loc];
-  T q = p * rc;
-  q = fused(fused(-q, c, p), rc, q);
-  return fused(fused(-q, c, p), rc, q);
+  T q = p * R.rc[loc];
+  q = fused(fused(-q, R.c2[loc], p), R.rc[loc], q);
+  return fused(fused(-q, R.c2[loc], p), R.rc[loc], q);
+}
+template <int DIM, typename T>
+__device__ inline T full_ghost(const SmallRobin<T>& R, int loc, T u) {
+  const T p = DIM == 3 ? (T)0 + u * R.c1[loc] : u * R.c1[loc];
+  return p / R.c2[loc];
 }
 template <int DIM, typename T>
 __device__ inline T small_ghost(const SmallRobin<T>& R, int loc, T u) {
-  if (((R.quick >> loc) & 1) && quick_range(u)) return quick_ghost<DIM>(R, loc, u);
-  const T p = DIM == 3 ? (T)0 + u * R.c1[loc] : u * R.c1[loc];
-  return p / R.c2[loc];
+  if (R.exact) return u * R.rc[loc];
+  if (R.quick && quick_range(u)) return quick_ghost<DIM>(R, loc, u);
+  return full_ghost<DIM>(R, loc, u);
 }
 
 // Slots of a level's colour arrays in LDS: `row` per row, `plane` per plane,
@@ -250,7 +255,6 @@ template <int DIM, bool DVAR, int CMODE, int N, typename T, int NC>
 __device__ inline void small_residuals(const T* E, int c, int v0, const Slots& S,
                                        const SmallCells<T, NC>& q, const SmallConst<T>& s,
                                        const SmallRobin<T>& R, T* res) {
-  constexpr int kAll = (1 << 2 * DIM) - 1;
   const T* o = E + (c ^ 1) * S.stride + S.pad;
   SmallNbr<T> n[N];
 #pragma unroll
@@ -273,18 +277,18 @@ __device__ inline void small_residuals(const T* E, int c, int v0, const Slots& S
     asm volatile("" : "+v"(fl));
     if (fl & 63) {
       const T uc = q.u[c][v0 + v];
-      if (R.exact == kAll) {
+      if (R.exact) {
 #pragma unroll
         for (int loc = 0; loc < 2 * DIM; ++loc)
           if (fl & (1 << loc)) n[v].v[loc] = uc * R.rc[loc];
-      } else if (R.quick == kAll && !__any(!quick_range(uc))) {
+      } else if (R.quick && !__any(!quick_range(uc))) {
 #pragma unroll
         for (int loc = 0; loc < 2 * DIM; ++loc)
           if (fl & (1 << loc)) n[v].v[loc] = quick_ghost<DIM>(R, loc, uc);
       } else {
 #pragma unroll
         for (int loc = 0; loc < 2 * DIM; ++loc)
-          if (fl & (1 << loc)) n[v].v[loc] = small_ghost<DIM>(R, loc, uc);
+          if (fl & (1 << loc)) n[v].v[loc] = full_ghost<DIM>(R, loc, uc);
       }
     }
   }
