@@ -111,8 +111,9 @@ void launch_box_side(const LevelGeom& L, const double* const* x, int g, int a, d
                      int fp32 = 0);
 
 // ---- levels that fit one work-group's LDS (box_small.hip) ----
-// Does one work-group hold the level (cells, coefficients of A's kind)?
-bool box_lds_fits(const BoxLevel& G, const BoxArrays& A);
+// Does one work-group hold the level (cells, coefficients of A's kind), and is
+// it the faster way to take that many sweeps?
+bool box_lds_pays(const BoxLevel& G, const BoxArrays& A, int sweeps);
 // `sweeps` red-black sweeps in one launch, homogeneous Robin ghosts: u from
 // uin (nullptr: 0) to e0 or e1 by the parity of the sweeps done.  With check,
 // K's early-exit test runs after every sweep (tol, stop, sweeps, maxres_out

@@ -64,17 +64,35 @@ k_box_lds_rbgs(BoxLevel G, BoxArraysT<T> A, SmallRobin<T> R, const T* uin, T* e0
   }
 }
 
-// Units per thread and colour of k_box_lds_rbgs, 0 if the grid-parallel sweep
-// is the better one.  Coefficients: what the registers of 512 threads hold,
-// 4096 cells in FP64 and 8192 in FP32.  Constant D and C: 4096 cells in 3-D
-// (16^3 2.5 us against 8.7; 20^3 spills and takes as long as the grid
-// launch's 8.3) and 8192 in 2-D (128 x 64 3.2 us against 4.5).
-int small_slots(const BoxLevel& G, bool coefs, bool fp32) {
+// Most units per thread and colour compiled in, where k_box_lds_rbgs is faster
+// than two sweeps per launch (box_pair.hip).  us per sweep with the early-exit
+// test, against that:
+//   coefficients: four, 15^3 D 4.4 (5.2), D and C 5.5 (5.3), 16^3 3.1 (5.0),
+//     4.3 (5.1), FP32 2.4 (5.1), 64 x 64 1.8 (2.9); eight spill, in 3-D up to
+//     211 registers, and take 11 (5.1) on 20^3, but 2-D FP32 2.5 (3.0) on 90 x 90;
+//   constant D and C: two, 16^3 2.6 (4.5), 64 x 64 1.5 (2.9); four, 90 x 90
+//     3.1 (3.0), FP32 2.1 (2.9).
+template <int DIM, typename T>
+constexpr int kSmallSlots(bool coefs) {
+  return DIM == 2 && sizeof(T) == 4 ? (coefs ? 8 : 4) : (coefs ? 4 : 2);
+}
+// A launch reads its coefficients once and pays for it over its sweeps: with
+// four units and more it takes 5 to 13 us longer to start than a pair, so
+// calls of few sweeps (two on 16^3: 53.5 against 48.4, 64 x 64 38.4 (33.3))
+// go to pairs.
+constexpr int kSmallFewSweeps = 16, kSmallFewSlots = 2;
+
+// Units per thread and colour of k_box_lds_rbgs for a call of that many
+// sweeps, 0 if it is not the better one.
+int small_slots(const BoxLevel& G, bool coefs, bool fp32, int sweeps) {
   const Slots S = slots_of(G);
   const int threads = kSmallThreads(coefs);
   int nc = 1;
   while (nc * threads < S.units) nc *= 2;
-  if (nc > (coefs ? (fp32 ? 8 : 4) : (G.dim == 3 ? 2 : 4))) return 0;
+  int most = G.dim == 3 ? kSmallSlots<3, double>(coefs)
+                        : (fp32 ? kSmallSlots<2, float>(coefs) : kSmallSlots<2, double>(coefs));
+  if (coefs && sweeps < kSmallFewSweeps) most = kSmallFewSlots;
+  if (nc > most) return 0;
   return S.count <= nc * threads && S.pad <= small_pad(nc * threads) ? nc : 0;
 }
 
@@ -84,7 +102,8 @@ struct LdsRun {
   static void run(const BoxLevel& G, const BoxArraysT<T>& A, const RobinDev& bc, const T* uin,
                   T* e0, T* e1, int sweeps, const BoxCheck& K, int check, hipStream_t s) {
     constexpr bool coefs = DVAR || CMODE == 2;
-    const int nc = small_slots(G, coefs, sizeof(T) == 4);
+    constexpr int most = kSmallSlots<DIM, T>(coefs);
+    const int nc = small_slots(G, coefs, sizeof(T) == 4, sweeps);
     const dim3 grid(1), block(small_threads(G, coefs));
     const SmallRobin<T> R = small_robin<T>(G, bc);
     auto go = [&](auto slots) {
@@ -94,9 +113,8 @@ struct LdsRun {
     };
     if (nc == 1) go(std::integral_constant<int, 1>{});
     else if (nc == 2) go(std::integral_constant<int, 2>{});
-    else if (nc == 4) go(std::integral_constant<int, 4>{});
-    else if (nc == 8 && coefs && sizeof(T) == 4)
-      go(std::integral_constant<int, coefs && sizeof(T) == 4 ? 8 : 4>{});
+    else if (nc == 4 && most >= 4) go(std::integral_constant<int, most >= 4 ? 4 : 2>{});
+    else if (nc == 8 && most >= 8) go(std::integral_constant<int, most >= 8 ? 8 : 2>{});
     else throw hipErrorInvalidValue;
     check_launch();
   }
@@ -104,8 +122,8 @@ struct LdsRun {
 
 }  // namespace
 
-bool box_lds_fits(const BoxLevel& G, const BoxArrays& A) {
-  return small_slots(G, A.D[0] != nullptr || A.cmode == 2, A.fp32 != 0) > 0;
+bool box_lds_pays(const BoxLevel& G, const BoxArrays& A, int sweeps) {
+  return small_slots(G, A.D[0] != nullptr || A.cmode == 2, A.fp32 != 0, sweeps) > 0;
 }
 
 void launch_box_lds_rbgs(const BoxLevel& G, const BoxArrays& A, const RobinDev& bc,

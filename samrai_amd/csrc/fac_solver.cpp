@@ -922,7 +922,7 @@ void CellPoissonFACOps::mgSweeps(int m, int n, bool zero_in) {
   K.stop = d_mg_flag;
   const sfac::RobinDev bc = robinDev();
   // a level that fits one work-group's LDS: all its sweeps in one launch
-  if (n > 0 && sfac::box_lds_fits(L.G, A)) {
+  if (n > 0 && sfac::box_lds_pays(L.G, A, n)) {
     sfac::launch_box_lds_rbgs(L.G, A, bc, zero_in ? nullptr : L.e[0], L.e[0], L.e[1], n, K, 0,
                               d_stream);
     return;
@@ -947,7 +947,7 @@ void CellPoissonFACOps::mgSweeps(int m, int n, bool zero_in) {
 // from buffer `from` (zero: from 0) to the other.
 bool CellPoissonFACOps::mgPair(int m) const {
   return d_box_variant < 0 && sfac::box_pair_pays(d_mg[m].G) &&
-         !sfac::box_lds_fits(d_mg[m].G, mgArrays(m));
+         !sfac::box_lds_pays(d_mg[m].G, mgArrays(m), 2);
 }
 
 void CellPoissonFACOps::mgPairSweeps(int m, int from, bool zero) {
@@ -1132,7 +1132,8 @@ int CellPoissonFACOps::smoothBox(PatchDataSet& e, const PatchDataSet& r, int num
   // a level that fits one work-group's LDS takes all its sweeps, with the
   // early-exit test after each, in one launch (a caller's tile shape asks for
   // the grid-parallel sweep)
-  const bool lds = num_sweeps > 0 && d_box_variant < 0 && sfac::box_lds_fits(G, A);
+  const bool lds =
+      num_sweeps > 0 && d_box_variant < 0 && sfac::box_lds_pays(G, A, num_sweeps);
   if (lds)
     sfac::launch_box_lds_rbgs(G, A, bc, B.e[0], B.e[0], B.e[1], num_sweeps, K, check, d_stream);
   // a larger one on which a launch is mostly latency takes two sweeps per

@@ -64,9 +64,9 @@ def solve(case, data, spec, keys, fused, variant, bits):
     return out, np.array(s.history()), count
 
 
-# slots per colour and thread 1, 2, 4 and 8, the last sizes that fit
-# (4096 cells with coefficients, 8192 without) and the first that do not,
-# odd rows, one-cell-wide and thin domains
+# slots per colour and thread 1, 2, 4 and (FP32 in 2-D) 8, the last sizes
+# that one work-group takes and the first that go to pairs, which calls of fewer
+# than 16 sweeps do from 4 slots on; odd rows, one-cell-wide and thin domains
 SIZES = [(3, 2, 2), (1, 5, 7), (9, 10, 11), (13, 17, 15), (16, 16, 16), (17, 16, 16), (32, 16, 16),
          (34, 16, 16), (2, 40, 40), (5, 3), (31, 23), (64, 64), (65, 64), (90, 91), (128, 64),
          (130, 64), (300, 9),
