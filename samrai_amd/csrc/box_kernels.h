@@ -80,8 +80,7 @@ struct BoxTile {
   int tx, ty, tz;
 };
 // Tile shapes compiled in (index = variant), per dimension.
-constexpr int kBoxTile16x4x4 = 9, kBoxTile16x8x4 = 10;  // 3-D
-constexpr int kBoxTile16x8 = 9;                         // 2-D
+constexpr int kBoxTile16x8x4 = 10;  // 3-D
 int box_tile_variants(int dim);
 BoxTile box_tile(int dim, int variant);
 

@@ -823,6 +823,7 @@ sfac::BoxArrays CellPoissonFACOps::gatherBox(PatchDataSet& e, const PatchDataSet
 namespace {
 constexpr int kMGPre = 2, kMGPost = 2, kMGSmallSweeps = 60, kMGLastSweeps = 64;
 constexpr int kMGDenseCycles = 4;  // V-cycles from which on the matrix pays
+constexpr int kMGSmallTileCells = 400000;  // mgVariant
 }
 
 void CellPoissonFACOps::releaseMG() {
@@ -960,15 +961,16 @@ void CellPoissonFACOps::mgPairSweeps(int m, int from, bool zero) {
   sfac::launch_box_pair(L.G, A, robinDev(), P, 2, d_stream);
 }
 
-// Tile shape of multigrid level m's sweeps: the tuned one on the finest level
-// (or the caller's); below it a sweep is latency, shortest with tiles small
-// enough for more work-groups than compute units (32^3 variable D: 16x4x4
-// 5.8 us, 16x8x8 7.9; 64^3: 16x8x4 7.6, 16x8x8 8.2, 16x4x4 8.3; 2-D 124 x 92:
-// 16x8 3.9, 16x16 4.1).
+// Tile shape of the sweeps of a multigrid level too large for two sweeps per
+// launch: the finest level's (tuned, or the caller's), but in 3-D a smaller one
+// where that leaves compute units without a tile.  us per sweep 64^3: 16x8x4 7.6,
+// 16x8x8 8.2; a coarse solve of ten V-cycles, FP32, second level 80 x 72 x 64:
+// 2044 with 16x8x4, 2184 with the finest level's; 96^3 3605 and 3562, 128^3
+// 6570 and 6474; 2-D 1024^2 (16x8 there) 4344 and 4117.
 int CellPoissonFACOps::mgVariant(int m) const {
-  if (m == 0 || d_box_variant >= 0) return d_box.variant;
-  if (d_h.dim() == 2) return sfac::kBoxTile16x8;
-  return mgCells(m) <= 100000 ? sfac::kBoxTile16x4x4 : sfac::kBoxTile16x8x4;
+  if (m == 0 || d_box_variant >= 0 || d_h.dim() == 2 || mgCells(m) > kMGSmallTileCells)
+    return d_box.variant;
+  return sfac::kBoxTile16x8x4;
 }
 
 int CellPoissonFACOps::mgCells(int m) const {
