@@ -278,12 +278,14 @@ int sfac_solver_set_algorithm_choice(sfac_solver* s, const char* choice);
 /* Execution choice with no reference counterpart (results are unchanged):
  * when the coarsest level of the solve tiles the physical domain exactly,
  * its red-black sweeps run colour-fused over one contiguous copy of the
- * level, one launch per sweep (the timing above then counts 24 / 48 B per
- * cell per launch).  on = 0 keeps the patch-wise colour passes.
+ * level, one launch per sweep or fewer (the timing above then counts a launch
+ * and 24 / 48 B per cell for every sweep).  on = 0 keeps the patch-wise colour passes.
  * tile_variant selects the LDS tile shape (0 .. sfac_fused_tile_variants-1),
  * or -1 (default) for the autotuner, which times every shape once per level
- * shape and keeps the fastest.  fused_coarsest_active / fused_tile_variant
- * report the path and shape in use after sfac_solver_initialize. */
+ * shape and keeps the fastest; small levels then take no tiles (all sweeps in
+ * one work-group, or two sweeps per launch).  fused_coarsest_active /
+ * fused_tile_variant report the path and shape in use after
+ * sfac_solver_initialize (shape -1: no tiles). */
 int sfac_solver_set_fused_coarsest(sfac_solver* s, int on, int tile_variant);
 int sfac_solver_fused_coarsest_active(sfac_solver* s, int* active);
 int sfac_solver_fused_tile_variant(sfac_solver* s, int* variant);
@@ -302,7 +304,7 @@ int sfac_solver_fused_tile_variant(sfac_solver* s, int* variant);
 int sfac_solver_set_fused_levels(sfac_solver* s, int on, int tile_variant);
 int sfac_solver_fused_level_variant(sfac_solver* s, int ln, int* variant);
 /* The autotuner's measured milliseconds per sweep of each tile shape (n = 0
- * when the shape was set explicitly). */
+ * when the shape was set explicitly or the sweeps take no tiles). */
 int sfac_solver_fused_tile_timings(sfac_solver* s, double* ms_per_sweep, int max, int* n);
 int sfac_fused_tile_variants(int dim);
 int sfac_fused_tile_shape(int dim, int variant, int* shape3);

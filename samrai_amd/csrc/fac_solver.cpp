@@ -361,8 +361,17 @@ void CellPoissonFACOps::setFusedCoarsest(bool on, int tile_variant) {
     fail("CellPoissonFACOps: tile variant out of range");
   d_box_enabled = on;
   d_box_variant = tile_variant;
-  if (d_box.ok) d_box.variant = tile_variant >= 0 ? tile_variant : tuneBoxVariant();
+  if (d_box.ok) chooseBoxVariant();
   ++d_generation;
+}
+
+// The tile shape of the coarsest level's sweeps: the caller's, or the tuned
+// one, or none where one work-group or two sweeps per launch take them (every
+// level that one work-group takes is small enough for those).
+void CellPoissonFACOps::chooseBoxVariant() {
+  d_box_timings.clear();
+  d_box.variant = d_box_variant;
+  if (d_box_variant < 0 && !sfac::box_pair_pays(d_box.G)) d_box.variant = tuneBoxVariant();
 }
 
 // Autotuner: time 8 back-to-back fused sweeps of every tile shape on the
@@ -769,7 +778,7 @@ void CellPoissonFACOps::setupBoxPath() {
       return;
     }
   }
-  B.variant = d_box_variant >= 0 ? d_box_variant : tuneBoxVariant();
+  chooseBoxVariant();
   if (d_coarse_choice == "mg" || d_coarse_choice == "hypre") setupMG();
 }
 

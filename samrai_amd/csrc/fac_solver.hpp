@@ -244,9 +244,10 @@ class CellPoissonFACOps : public FACOperatorStrategy {
   // fastest.
   void setFusedCoarsest(bool on, int tile_variant);
   bool fusedCoarsestActive() const { return d_box.ok && d_box_enabled; }
+  // -1: none in use (no such level, or its sweeps take no tiles)
   int fusedTileVariant() const { return d_box.ok ? d_box.variant : -1; }
   // the autotuner's measured time per sweep of every tile shape (ms; empty
-  // when the shape was given or came from the cache)
+  // when the shape was given or the sweeps take no tiles)
   const std::vector<float>& fusedTileTimings() const { return d_box_timings; }
   // Colour-fused sweeps on the levels above the coarsest (level_fused.h):
   // on by default where a level qualifies (3-D, non-negative indices,
@@ -336,12 +337,13 @@ class CellPoissonFACOps : public FACOperatorStrategy {
     double* C = nullptr;
     double* slots = nullptr;
     int* mismatch = nullptr;
-    int variant = 0;
+    int variant = -1;
     int fp32 = 0;  // arrays hold float (mixed-precision coarse solve)
   } d_box;
   bool d_box_enabled = true;
   bool d_coarse_fp32 = false;
   int tuneBoxVariant();
+  void chooseBoxVariant();
   std::vector<float> d_box_timings;
   sfac::BoxArrays gatherBox(pdat::PatchDataSet& e, const pdat::PatchDataSet& r);
   // geometric multigrid on the single-rectangle coarsest level

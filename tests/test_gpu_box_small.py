@@ -100,6 +100,35 @@ def test_lds_sweeps_are_bit_identical(gpu_lib, n, spec):
                 np.testing.assert_array_equal(a, b)
 
 
+@pytest.mark.parametrize("n,tiled", [((64, 64), False), ((53, 53, 53), False),
+                                     ((56, 55, 54), True), ((512, 600), True)],
+                         ids=lambda v: "x".join(map(str, v)) if isinstance(v, tuple) else str(v))
+def test_tile_shape_is_tuned_only_where_tiles_run(gpu_lib, n, tiled):
+    """A level whose sweeps run in one work-group or two per launch reports no
+    tile shape and times none at set-up; a larger one, or one with a shape of
+    the caller's, does."""
+    from samrai_amd import fac
+    print("tile shape", n, flush=True)
+    dim = len(n)
+    h = fac.PatchHierarchy(dim, (0,) * dim, [v - 1 for v in n], [0.0] * 3, [1.0] * 3)
+    cut = n[1] // 4 * 2  # a patch is at most 512 cells wide
+    h.add_level(1, [((0,) * dim, (n[0] - 1, cut - 1) + tuple(v - 1 for v in n[2:])),
+                    ((0, cut, 0)[:dim], tuple(v - 1 for v in n))])
+    h.finalize()
+    u, f = fac.PatchData(h, 1), fac.PatchData(h, 0)
+    s = fac.CellPoissonFACSolver(h, max_cycles=1)
+    s.set_dirichlet(0.0)
+    s.initialize_solver_state(u, f)
+    assert s.fused_coarsest_active()
+    shapes = len(fac.fused_tile_shapes(dim))
+    assert len(s.fused_tile_timings()) == (shapes if tiled else 0)
+    assert 0 <= s.fused_tile_variant() < shapes if tiled else s.fused_tile_variant() == -1
+    s.set_fused_coarsest(True, 2)
+    assert s.fused_tile_variant() == 2 and s.fused_tile_timings() == []
+    s.set_fused_coarsest(True)
+    assert (s.fused_tile_variant() >= 0) == tiled
+
+
 MG = dict(max_cycles=6, residual_tol=1e-300, relative_residual_tol=1e-300, num_pre_sweeps=1,
           num_post_sweeps=1, coarse_solver_choice="mg", coarse_solver_tolerance=1e-300,
           coarse_solver_max_iterations=3)
