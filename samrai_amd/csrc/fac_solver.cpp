@@ -831,7 +831,14 @@ sfac::BoxArrays CellPoissonFACOps::gatherBox(PatchDataSet& e, const PatchDataSet
 
 namespace {
 constexpr int kMGPre = 2, kMGPost = 2, kMGSmallSweeps = 60, kMGLastSweeps = 64;
-constexpr int kMGDenseCycles = 4;  // V-cycles from which on the matrix pays
+// A coarse solve forms the lower levels' matrix (mg_bottom.hip) when it may take
+// this many V-cycles and its tolerance asks for more than one (a V-cycle
+// reduces the residual 20 to 50 times).  us per coarse solve and cycle, matrix and
+// one work-group, on 20^3 with variable D, whose lower part has 1000 cells:
+// tolerance 0.5 575, 310; 0.05 587, 349; 0.01 612, 424; 1e-4 650, 541; 1e-6
+// 716, 748; on 32^3 (512 cells): 370, 361; 390, 396; 428, 462; 491, 564; 588, 734.
+constexpr int kMGDenseCycles = 4;
+constexpr double kMGDenseTol = 1e-2;
 constexpr int kMGSmallTileCells = 400000;  // mgVariant
 }
 
@@ -1055,10 +1062,9 @@ void CellPoissonFACOps::solveBoxMG(PatchDataSet& e, const PatchDataSet& r) {
   // ||r||^2 into d_mg_scal[1] and the relative-residual test
   sfac::launch_mg_sum_check(d_mg_partial, P, d_mg_scal, d_mg_scal, tol, -1, d_mg_flag,
                             d_mg_flag + 1, d_mg_scal + 2, d_stream);
-  // the lower levels' matrix takes about as long as two passes through them;
   // formed per solve, since the caller may change the coefficients between
   // solves (level 0 starts from the last V-cycle's error, not from 0)
-  d_mg_use_dense = d_mg_dense && d_coarse_max >= kMGDenseCycles;
+  d_mg_use_dense = d_mg_dense && d_coarse_max >= kMGDenseCycles && tol <= kMGDenseTol;
   if (d_mg_use_dense) mgBottom(mgCells(d_mg_bottom), d_mg_dense);
   for (int it = 0; it < d_coarse_max; ++it) {
     mgVcycle(0);

@@ -8,10 +8,11 @@
 // same coefficients.  So a coarse solve that may take several V-cycles forms B
 // once, one work-group per column (k_mg_bottom on the unit vectors, all
 // columns at once), and a V-cycle's lower part is one matrix-vector product.
-// In one work-group the lower part of a 128^3 level's V-cycle took 97 us a
-// cycle from 16^3 on, as launches per step about 70 us from 8^3 on; the product
-// takes 4.  The FAC solve of the 54 M cell hierarchy goes from 309 to 296 ms,
-// of a 2-D one whose smallest grid is 31 x 23 from 37.8 to 29.3 ms.
+// In one work-group, as a coarse solve of few V-cycles takes it, the lower part
+// from 8^3 on is 45 us a V-cycle (as launches per step 76), from 10^3 on 81 us
+// (105); the product takes 4.  The FAC solve of the 54 M cell hierarchy goes from
+// 309 to 296 ms with it, of a 2-D one whose smallest grid is 31 x 23 from 37.8 to
+// 29.3 ms.
 #include <cstddef>
 #include <type_traits>
 
