@@ -129,36 +129,75 @@ def test_tile_shape_is_tuned_only_where_tiles_run(gpu_lib, n, tiled):
     assert (s.fused_tile_variant() >= 0) == tiled
 
 
-MG = dict(max_cycles=6, residual_tol=1e-300, relative_residual_tol=1e-300, num_pre_sweeps=1,
-          num_post_sweeps=1, coarse_solver_choice="mg", coarse_solver_tolerance=1e-300,
-          coarse_solver_max_iterations=3)
-
-
+MG = dict(residual_tol=1e-300, relative_residual_tol=1e-300, num_pre_sweeps=1,
+          num_post_sweeps=1, coarse_solver_choice="mg")
 # lower parts of one to six levels, starting on the finest or a coarser level,
-# first levels of one and of four cells a thread, halving that stops at odd
-# extents (the last grid's 64 sweeps) or at the smallest edge, a level too
-# large for the lower part that cannot be halved (33^3: none)
-@pytest.mark.parametrize("spec", [dict(dvar=False), dict(dvar=True, cmode=2, robin=True),
-                                  dict(dvar=True, cmode=1, cconst=-0.3)],
-                         ids=["constD", "varD-varC-robin", "varD-constC"])
-@pytest.mark.parametrize("n", [(4, 4, 4), (8, 8, 8), (12, 20, 8), (16, 16, 16), (24, 16, 18),
-                               (33, 33, 33), (40, 32, 48), (4, 6), (64, 64), (62, 46), (96, 40),
-                               (256, 128)], ids=lambda n: "x".join(map(str, n)))
-def test_multigrid_lower_part_matches_oracle(gpu_lib, n, spec):
-    """Residual history and solution of a one-level FAC solve with the
-    multigrid coarse solver against the oracle's multigrid: the values of every
-    level operation are the same and only the norms' sums are ordered
-    differently, so both agree to 1e-10 as the other multigrid solves do."""
+# first levels of one and of four cells a thread and of exactly 1024 cells,
+# halving that stops at odd extents (the last grid's 64 sweeps) or at the
+# smallest edge, a level too large for the lower part that cannot be halved
+# (33^3: none)
+MG_SIZES = [(4, 4, 4), (8, 8, 8), (12, 20, 8), (16, 16, 16), (24, 16, 18), (20, 20, 20),
+            (32, 16, 16), (33, 33, 33), (40, 32, 48), (4, 6), (64, 64), (62, 46), (66, 62),
+            (96, 40), (128, 32), (256, 128)]
+MG_SPECS = [dict(dvar=False), dict(dvar=True, cmode=2, robin=True),
+            dict(dvar=True, cmode=1, cconst=-0.3),
+            dict(dvar=False, cmode=1, cconst=-0.7, robin=True)]
+MG_IDS = ["constD", "varD-varC-robin", "varD-constC", "constD-constC-robin"]
+
+
+def mg_pair(n, spec, cycles, tol, max_cycles=6):
     case = one_level(*n)
     spec = dict(spec)
     if spec.pop("robin", False):
         spec["bc"] = hc.bc_robin(case["dim"])
     data = hc.make_data(case, seed=sum(n))
-    print("multigrid lower part", case["name"], spec, flush=True)
-    pr = hc.Pair(case, MG, data, **spec)
+    print("multigrid lower part", case["name"], spec, cycles, tol, flush=True)
+    return hc.Pair(case, dict(MG, max_cycles=max_cycles, coarse_solver_max_iterations=cycles,
+                              coarse_solver_tolerance=tol), data, **spec)
+
+
+# the lower part in one work-group (at most three V-cycles a coarse solve, or a
+# tolerance that one or two meet) and as a matrix
+@pytest.mark.parametrize("cycles,tol", [(3, 1e-300), (10, 1e-300), (10, 0.05)],
+                         ids=["three", "matrix", "loose"])
+@pytest.mark.parametrize("spec", MG_SPECS, ids=MG_IDS)
+@pytest.mark.parametrize("n", MG_SIZES, ids=lambda n: "x".join(map(str, n)))
+def test_multigrid_lower_part_matches_oracle(gpu_lib, n, spec, cycles, tol):
+    """Residual history and solution of a one-level FAC solve with the
+    multigrid coarse solver against the oracle's multigrid: the values of every
+    level operation are the same and only the norms' sums are ordered
+    differently, so both agree to 1e-10 as the other multigrid solves do.
+
+    After ten V-cycles a residual is soon all rounding.  A cell's is a sum of
+    2 dim fluxes D (u - u') / dx^2, each rounded a few times in relation to
+    D u / dx^2, and the matrix rounds in other places than the steps it stands
+    for: 16 roundings of the stencil's 4 D sum(1 / dx^2) max |u|."""
+    pr = mg_pair(n, spec, cycles, tol)
     pr.s.solve_system(pr.u, pr.f)
     _, it, _, hist = pr.o.solve()
     assert pr.s.number_of_iterations() == it
-    scale = max(hist)
-    np.testing.assert_allclose(pr.s.history(), hist, rtol=1e-10, atol=1e-13 * scale)
+    atol = 1e-13 * max(hist)
+    if cycles == 10 and tol < 1e-10:
+        D = np.exp(0.8) if spec["dvar"] else 1.0
+        u = max(np.abs(pr.o.get("u", 0, p)).max() for p in range(pr.npatch(0)))
+        atol = max(atol, 16 * 2.0 ** -53 * 4 * D * sum(v * v for v in n) * u)
+        assert atol <= 1e-9  # the first residual is of order 1
+    np.testing.assert_allclose(pr.s.history(), hist, rtol=1e-10, atol=atol)
     pr.compare(pr.u, "u", interior_only=True, rtol=1e-10)
+
+
+@pytest.mark.parametrize("spec", MG_SPECS, ids=MG_IDS)
+@pytest.mark.parametrize("n", [n for n in MG_SIZES if np.prod(n) > 1024 and n != (33, 33, 33)],
+                         ids=lambda n: "x".join(map(str, n)))
+def test_multigrid_matrix_in_fp32(gpu_lib, n, spec):
+    """The FP32 coarse solve with its lower levels as a matrix: every FAC cycle
+    reduces the FP64 residual by a coarse solve to 1e-6 or by ten V-cycles (30
+    times on 66 x 62, whose last grid 33 x 31 takes 64 sweeps), so ten of them
+    reach the FP64 oracle's solution to 1e-8 of max |u|."""
+    pr = mg_pair(n, spec, 10, 1e-300, max_cycles=10)
+    pr.s.set_coarse_precision(32)
+    pr.s.solve_system(pr.u, pr.f)
+    pr.o.solve()
+    hist = pr.s.history()
+    assert hist[-1] <= 1e-9 * hist[0]
+    pr.compare(pr.u, "u", interior_only=True, rtol=1e-8)
