@@ -478,20 +478,14 @@ __device__ inline T mg_restrict_value(const BoxLevel& Gf, const BoxArraysT<T>& A
   return sum * (T)(DIM == 3 ? 0.125 : 0.25);
 }
 
-// Cell (i, j, k) of linear index t of a box n0 x n1 x ...; levels below 2^32
-// cells divide in 32 bits (a 64-bit division is a routine of over 100
-// instructions, as long as the rest of these kernels' work on a cell).
-__device__ inline void mg_cell(long t, long ncells, int n0, int n1, int& i, int& j, int& k) {
-  if (ncells <= 0xffffffffl) {
-    const unsigned row = (unsigned)t / (unsigned)n0;
-    i = (int)((unsigned)t - row * (unsigned)n0);
-    k = (int)(row / (unsigned)n1);
-    j = (int)(row - (unsigned)k * (unsigned)n1);
-  } else {
-    i = (int)(t % n0);
-    j = (int)((t / n0) % n1);
-    k = (int)(t / ((long)n0 * n1));
-  }
+// Cell (i, j, k) of linear index t of a box n0 x n1 x ... (a level has at most
+// 2^30 cells: setupBoxPath).  In 32 bits: a 64-bit division is a routine of over
+// 100 instructions, as long as the rest of these kernels' work on a cell.
+__device__ inline void mg_cell(unsigned t, int n0, int n1, int& i, int& j, int& k) {
+  const unsigned row = t / (unsigned)n0;
+  i = (int)(t - row * (unsigned)n0);
+  k = (int)(row / (unsigned)n1);
+  j = (int)(row - (unsigned)k * (unsigned)n1);
 }
 
 // fc = mean over the 2^dim children of the fine residual (one thread per
@@ -505,7 +499,7 @@ k_mg_restrict_residual(BoxLevel Gf, BoxArraysT<T> A, RobinDev bc, const T* u, Bo
   for (long t = (long)blockIdx.x * kThreads + threadIdx.x; t < nc;
        t += (long)gridDim.x * kThreads) {
     int I, J, K;
-    mg_cell(t, nc, Gc.n[0], Gc.n[1], I, J, K);
+    mg_cell((unsigned)t, Gc.n[0], Gc.n[1], I, J, K);
     fc[t] = mg_restrict_value<DIM, DVAR, CMODE>(Gf, A, bc, u, I, J, K);
   }
 }
@@ -526,7 +520,7 @@ k_mg_prolong_add(BoxLevel Gc, RobinDev bc, const T* ec, BoxLevel Gf, T* ef, cons
   for (long t = (long)blockIdx.x * kThreads + threadIdx.x; t < np;
        t += (long)gridDim.x * kThreads) {
     int I, j, k;
-    mg_cell(t, np, Gc.n[0], Gf.n[1], I, j, k);
+    mg_cell((unsigned)t, Gc.n[0], Gf.n[1], I, j, k);
     const int J = j >> 1, K = k >> 1;
     const int Js = J + ((j & 1) ? 1 : -1), Ks = K + ((k & 1) ? 1 : -1);
     const T e0 = ef[2 * t], e1 = ef[2 * t + 1];
@@ -632,7 +626,7 @@ k_mg_sumsq(BoxLevel G, BoxArraysT<T> A, RobinDev bc, const T* u, const T* x, dou
       v = (double)x[t];
     } else {
       int i, j, k;
-      mg_cell(t, n, G.n[0], G.n[1], i, j, k);
+      mg_cell((unsigned)t, G.n[0], G.n[1], i, j, k);
       v = (double)mg_residual<DIM, DVAR, CMODE>(G, A, bc, u, i, j, k);
     }
     acc += v * v;
