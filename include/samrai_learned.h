@@ -54,8 +54,8 @@ size_t sfac_conv3x3x3_wgrad_partial_size(int nblocks);
 /* No counterpart in the reference: the weight gradient above for callers that
  * cannot allocate device memory (code under HIP graph capture, tight serving
  * or training loops, harnesses that forbid hipMalloc).  It allocates nothing:
- * the per-wave slabs live in a static device array of the library, one per
- * GPU, 7 MiB, held until the process ends; its address is looked up for the
+ * the work-groups' slabs live in a static device array of the library, one per
+ * GPU, 1.75 MiB, held until the process ends; its address is looked up for the
  * current device on the first call there (the stream must belong to the
  * current device).  nblocks <= SFAC_WGRAD_NOALLOC_MAX_BLOCKS, larger counts
  * are rejected with an error.  Results are bit-identical to

@@ -1067,17 +1067,25 @@ T* dalloc(size_t n) {
 // block: quarters of a block while whole ones would leave compute units idle,
 // at most two work-groups per compute unit, which then take several.
 constexpr int kWgradGroups = 512;
-int wgrad_slabs(int nblocks) { return nblocks < 128 ? 4 : 1; }
-int wgrad_groups(int nblocks) { return std::min(nblocks * wgrad_slabs(nblocks), kWgradGroups); }
+constexpr int wgrad_slabs(int nblocks) { return nblocks < 128 ? 4 : 1; }
+constexpr int wgrad_groups(int nblocks) {
+  return std::min(nblocks * wgrad_slabs(nblocks), kWgradGroups);
+}
 
-// Per-wave gradient slabs of the allocation-free weight gradient
+// Gradient slabs, one per work-group, of the allocation-free weight gradient
 // (sfac_conv3x3x3_wgrad_bf16_noalloc): one array per GPU, held until the
 // process ends.  Host code never passes `scratch` itself to a kernel (on the
 // host it names a stand-in, not device memory): it passes the address that
 // hipGetSymbolAddress returns for the current device.
 constexpr int NOALLOC_MAX_BLOCKS = SFAC_WGRAD_NOALLOC_MAX_BLOCKS;
-constexpr size_t NOALLOC_FLOATS = (size_t)NOALLOC_MAX_BLOCKS * 16 * GSZ;  // 7 MiB
-static_assert(NOALLOC_MAX_BLOCKS < 128, "four slabs a block, 16 fit");
+constexpr int NOALLOC_SLABS = 4 * NOALLOC_MAX_BLOCKS;
+constexpr size_t NOALLOC_FLOATS = (size_t)NOALLOC_SLABS * GSZ;  // 1.75 MiB
+constexpr bool noalloc_slabs_fit() {
+  for (int n = 1; n <= NOALLOC_MAX_BLOCKS; ++n)
+    if (wgrad_groups(n) > NOALLOC_SLABS) return false;
+  return true;
+}
+static_assert(noalloc_slabs_fit(), "a slab for every work-group");
 __device__ __align__(256) float scratch[NOALLOC_FLOATS];
 
 constexpr int kMaxDevices = 64;
@@ -1373,7 +1381,7 @@ int sfac_conv3x3x3_wgrad_bf16_noalloc(const uint16_t* x, const uint16_t* gz, flo
       hipLaunchKernelGGL(k_zero_f32, dim3((GSZ + 255) / 256), dim3(256), 0, stream, grad, GSZ);
       return;
     }
-    // every wave of k_wgrad writes its whole slab, so nothing needs clearing
+    // every work-group of k_wgrad writes its whole slab, so nothing needs clearing
     launch_wgrad(x, gz, scratch_on_current_device(), grad, nblocks, stream);
   });
 }
