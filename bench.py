@@ -215,9 +215,10 @@ def smoother_rate(s, deck, ln, sweeps):
 
 MFMA_BF16_PEAK_TFLOPS = 2500.0
 # multiply-adds per cell of the network as specified (2 -> 16 -> 16 -> 1
-# channels, 27 taps); the kernels pad every layer to 16 x 16 channels
+# channels, 27 taps), and as the forward kernel issues them: per 16 cells, 2, 15
+# and 2 matrix products of 16 x 16 with K = 32 for the three layers
 LEARNED_MACS_PER_CELL = 27 * (2 * 16 + 16 * 16 + 16 * 1)
-LEARNED_PADDED_MACS_PER_CELL = 27 * 16 * 16 * 3
+LEARNED_PADDED_MACS_PER_CELL = (2 + 15 + 2) * 16 * 32
 
 
 def learned_section(torch, seeds, steps, batch, log=print, n=128, cycles=(1, 2, 3, 4, 5, 6, 7, 8)):
@@ -269,7 +270,8 @@ def learned_section(torch, seeds, steps, batch, log=print, n=128, cycles=(1, 2, 
     gs = [(torch.linalg.vector_norm(SL.block_sor(torch, tst["r"], tst["dxf"], tst["dyf"],
                                                  tst["dzf"], h, k, 1.0) - tst["e"]) / ne).item()
           for k in (1, 2, 4)]
-    # matrix-core rate of the forward pass (three conv launches) on the test blocks
+    # matrix-core rate of the forward pass (features, then one launch for the
+    # three layers) on the test blocks
     rb, lb = tst["r"], tst["logd"]
     nb = rb.shape[0]
     net.forward(rb, lb, h)
@@ -404,7 +406,7 @@ def learned_section(torch, seeds, steps, batch, log=print, n=128, cycles=(1, 2, 
                  "block error equation (zero Dirichlet on the block faces, 400 SOR sweeps)"
                  % (",".join(str(c) for c in cycles), n),
         network="3x3x3 conv 2->16->16->1, ReLU, BF16 weights/activations, FP32 accumulation "
-                "(v_mfma_f32_16x16x16_bf16), Adam on FP32 master weights",
+                "(v_mfma_f32_16x16x32_bf16), Adam on FP32 master weights",
         train_blocks=int(cat["r"].shape[0]), train_seeds=seeds, test_blocks=int(tst["r"].shape[0]),
         pair_generation_s=round(gen_s, 2), train_steps=steps, batch_blocks=batch,
         train_s=round(train_s, 3),
@@ -419,7 +421,7 @@ def learned_section(torch, seeds, steps, batch, log=print, n=128, cycles=(1, 2, 
         roofline=dict(bound="mfma", achieved=round(alg_tflops, 2), peak=MFMA_BF16_PEAK_TFLOPS,
                       unit="TFLOP/s", frac=round(alg_tflops / MFMA_BF16_PEAK_TFLOPS, 5),
                       padded_tflops=round(padded_tflops, 2),
-                      kernel="k_conv (3 launches, forward)",
+                      kernel="k_features, k_forward (the forward pass)",
                       flops_per_cell=2 * LEARNED_MACS_PER_CELL))
     net.close()
     return out

@@ -7,7 +7,7 @@
 // it grown by two, red by one, black on the tile; what neighbouring tiles
 // compute too comes from the same inputs in the same expression order, so the
 // values are those of two k_box_rbgs launches bit for bit.  The idle units pay
-// for the redundant cells (5.4 staged coefficient cells per owned one at
+// for the redundant cells (4.4 cells' coefficients loaded per owned one at
 // 8x8x8).  A cell's coefficients are read and its diagonal inverted once for
 // both sweeps, and the physical ghosts are formed inside the updates (the cell
 // is its face ghost's only interior neighbour).
