@@ -60,11 +60,19 @@ struct BoxArraysT {
   double cconst;
 };
 
-// Early-exit test of the sweep before this launch.  slots: three words
+// Early-exit test of the sweep before this launch.  slots: three slots
 // (nullptr without a tolerance); sweep s raises slot s % 3 to the max
 // |residual| over the last patch (an atomic max of the bit patterns, which
 // order like the values for non-negative doubles), reads slot (s + 2) % 3
 // (the previous sweep's) and clears slot (s + 1) % 3 for the next sweep.
+// A slot has eight words, on lines of their own, a work-group raising the one
+// that its index picks: hundreds of work-groups raising one word wait for each
+// other, and looking at the word first costs a round trip.  us per sweep, FP64,
+// with one word, one looked at first, eight: 128^3 in one patch 34.4, 29.5,
+// 19.1; D per face 37.5, 41.3, 31.0; 64^3 9.9, 8.5, 8.6; 128^3 with a last patch
+// of 64^3 18.1, 20.1, 18.4; D per face 29.0, 31.0, 29.6.
+constexpr int kCheckWords = 8, kCheckLine = 16;
+constexpr int kCheckSlot = kCheckWords * kCheckLine, kCheckSize = 3 * kCheckSlot;
 struct BoxCheck {
   unsigned long long* slots;
   int tlo[3], tn[3];    // tile range of the last patch

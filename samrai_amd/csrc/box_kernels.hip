@@ -40,8 +40,32 @@ __device__ inline double block_max(double v, double* wm) {
   return v;
 }
 
+// Value of the lane that CTRL (a data-parallel primitive's control) names.
+template <int CTRL>
+__device__ inline double lane_value(double v) {
+  const long long b = __double_as_longlong(v);
+  const int lo = __builtin_amdgcn_update_dpp(0, (int)b, CTRL, 0xf, 0xf, true);
+  const int hi = __builtin_amdgcn_update_dpp(0, (int)(b >> 32), CTRL, 0xf, 0xf, true);
+  return __longlong_as_double(((long long)hi << 32) | (unsigned int)lo);
+}
+
+// Largest |residual| of the sweep that raised slot s, the same in every lane: a
+// lane reads one word of the slot (one load for all; read in turn they cost
+// 0.4 us), then the maximum over eight lanes.
+__device__ inline double slot_max(const unsigned long long* slots, int s) {
+  static_assert(kCheckWords == 8, "three steps");
+  double m = __longlong_as_double(
+      (long long)slots[s * kCheckSlot + threadIdx.x % kCheckWords * kCheckLine]);
+  m = fmax(m, lane_value<0xb1>(m));   // neighbours in a pair (quad_perm 1, 0, 3, 2)
+  m = fmax(m, lane_value<0x4e>(m));   // the other pair of four (quad_perm 2, 3, 0, 1)
+  m = fmax(m, lane_value<0x141>(m));  // the other four of eight (row_half_mirror)
+  const long long b = __double_as_longlong(m);
+  return __longlong_as_double(((long long)__builtin_amdgcn_readfirstlane((int)(b >> 32)) << 32) |
+                              (unsigned int)__builtin_amdgcn_readfirstlane((int)b));
+}
+
 // Early-exit test of the previous sweep (see BoxCheck).  Every wave reads
-// the stop flag and the previous sweep's max-residual word itself (no
+// the stop flag and the previous sweep's max-residual words itself (no
 // barrier): all read the same words and take the same decision (a stop that
 // work-group 0 records during this sweep follows from the same test), and
 // work-group 0 records it.  true: skip this sweep.
@@ -49,10 +73,10 @@ __device__ inline bool stop_sweep(const BoxCheck& K, int b) {
   if (!K.stop) return false;
   bool stop;
   if (K.slots && K.sweep > 0) {
-    // both words are read unconditionally, so that their loads are in
-    // flight together (one memory round trip before the decision)
+    // all are read unconditionally, so that their loads are in flight
+    // together (one memory round trip before the decision)
     const int flag = *K.stop;
-    const double m = __longlong_as_double((long long)K.slots[(K.sweep + 2) % 3]);
+    const double m = slot_max(K.slots, (K.sweep + 2) % 3);
     const bool now = !(m > K.tol);
     stop = (flag != 0) | now;
     if (flag == 0 && now && b == 0 && threadIdx.x == 0) {
@@ -64,7 +88,8 @@ __device__ inline bool stop_sweep(const BoxCheck& K, int b) {
     stop = *K.stop != 0;
   }
   // the slot the next sweep raises (its last reader was the previous sweep)
-  if (!stop && K.slots && b == 0 && threadIdx.x == 0) K.slots[(K.sweep + 1) % 3] = 0ull;
+  if (!stop && K.slots && b == 0 && threadIdx.x < kCheckWords)
+    K.slots[(K.sweep + 1) % 3 * kCheckSlot + threadIdx.x * kCheckLine] = 0ull;
   return stop;
 }
 
@@ -254,14 +279,15 @@ k_box_rbgs(BoxLevel G, BoxArraysT<T> A, RobinDev bc, int homogeneous, BoxCheck K
     if (meets) {  // uniform over the work-group
       mr = block_max(mr, wm);
       if (threadIdx.x == 0)
-        raise_max(K.slots + K.sweep % 3, mr);
+        atomicMax(K.slots + K.sweep % 3 * kCheckSlot + b % kCheckWords * kCheckLine,
+                  (unsigned long long)__double_as_longlong(mr));
     }
   }
 }
 
 __global__ void __launch_bounds__(kThreads) k_box_final_check(BoxCheck K, int nsweeps) {
   if (*K.stop) return;  // stopped early: already recorded
-  const double m = __longlong_as_double((long long)K.slots[(nsweeps - 1) % 3]);
+  const double m = slot_max(K.slots, (nsweeps - 1) % 3);
   if (threadIdx.x == 0) {
     *K.sweeps = nsweeps;
     if (K.maxres_out) *K.maxres_out = m;

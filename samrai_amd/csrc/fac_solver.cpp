@@ -751,8 +751,9 @@ void CellPoissonFACOps::setupBoxPath() {
   hip_check(hipMalloc(&B.e[0], sizeof(double) * vol), "hipMalloc(box e)");
   hip_check(hipMalloc(&B.e[1], sizeof(double) * vol), "hipMalloc(box e)");
   hip_check(hipMalloc(&B.r, sizeof(double) * vol), "hipMalloc(box r)");
-  // early-exit maxima of three consecutive sweeps (BoxCheck) or pairs (PairCheck)
-  hip_check(hipMalloc(&B.slots, sizeof(double) * 6), "hipMalloc(box slots)");
+  // early-exit maxima of three consecutive sweeps (BoxCheck) or pairs (six words,
+  // PairCheck)
+  hip_check(hipMalloc(&B.slots, sizeof(double) * sfac::kCheckSize), "hipMalloc(box slots)");
   hip_check(hipMalloc(&B.mismatch, sizeof(int)), "hipMalloc(box flag)");
   if (d_spec.cMode() == 2) hip_check(hipMalloc(&B.C, sizeof(double) * vol), "hipMalloc(box C)");
   B.ok = true;
@@ -1131,7 +1132,7 @@ int CellPoissonFACOps::smoothBox(PatchDataSet& e, const PatchDataSet& r, int num
   const bool check = tol >= 0.0;
   if (check) {
     sfac::launch_fill_int(d_stop, 2, 0, d_stream);
-    sfac::launch_fill(B.slots, 3, 0.0, d_stream);  // the first sweep's slot
+    sfac::launch_fill(B.slots, sfac::kCheckSize, 0.0, d_stream);  // the first sweep's slot
     K.stop = d_stop;
     K.sweeps = d_stop + 1;
     K.maxres_out = d_scalars + 1;
