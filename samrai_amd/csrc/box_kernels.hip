@@ -491,11 +491,17 @@ __device__ inline T mg_residual(const BoxLevel& G, const BoxArraysT<T>& A, const
 }
 
 // Mean over the 2^dim children of coarse cell (I, J, K) of the fine
-// residual (children summed in i, j, k order).
+// residual (children summed in i, j, k order).  In 3-D four children's loads
+// in flight and a third wave per SIMD are better than eight, but not with FP64
+// face coefficients (kRestrictAll): us a call over 64^3 to 256^3 levels, four and
+// eight, D per face FP64 79, 74, FP32 48, 54, constant D 41, 42.
+template <int DIM, bool DVAR, typename T>
+constexpr bool kRestrictAll = DIM == 2 || (DVAR && sizeof(T) == 8);
 template <int DIM, bool DVAR, int CMODE, typename T>
 __device__ inline T mg_restrict_value(const BoxLevel& Gf, const BoxArraysT<T>& A,
                                       const RobinDev& bc, const T* u, int I, int J, int K) {
   T sum = 0;
+#pragma unroll (kRestrictAll<DIM, DVAR, T> ? 2 : 1)
   for (int c2 = 0; c2 < (DIM == 3 ? 2 : 1); ++c2)
     for (int c1 = 0; c1 < 2; ++c1)
       for (int c0 = 0; c0 < 2; ++c0)
@@ -525,7 +531,16 @@ k_mg_restrict_residual(BoxLevel Gf, BoxArraysT<T> A, RobinDev bc, const T* u, Bo
   for (long t = (long)blockIdx.x * kThreads + threadIdx.x; t < nc;
        t += (long)gridDim.x * kThreads) {
     int I, J, K;
-    mg_cell((unsigned)t, Gc.n[0], Gc.n[1], I, J, K);
+    if (DIM == 3 && kRestrictAll<DIM, DVAR, T>) {
+      // 64-bit divisions: with mg_cell all of the eight children's loads go
+      // ahead of their uses, in so many registers that one wave per SIMD is
+      // left (91 us a call)
+      I = (int)(t % Gc.n[0]);
+      J = (int)((t / Gc.n[0]) % Gc.n[1]);
+      K = (int)(t / ((long)Gc.n[0] * Gc.n[1]));
+    } else {
+      mg_cell((unsigned)t, Gc.n[0], Gc.n[1], I, J, K);
+    }
     fc[t] = mg_restrict_value<DIM, DVAR, CMODE>(Gf, A, bc, u, I, J, K);
   }
 }
